@@ -65,6 +65,7 @@ int fail(int code, const char* fmt, ...) {
 struct SizeFns {
   hipFunction_t row_fwd = nullptr, row_inv = nullptr, coly_fwd = nullptr, coly_inv = nullptr;
   hipFunction_t colz_fwd = nullptr, colz_inv = nullptr, colz_conv = nullptr;
+  hipFunction_t cube_fwd = nullptr, cube_inv = nullptr, cube_conv = nullptr;  // N in {8, 16}: a cube per work-group
   hipFunction_t plane_fwd = nullptr, plane_inv = nullptr;                 // N in {32, 64, 128}
   hipFunction_t coly_fwd_zb = nullptr, coly_inv_zb = nullptr, colz_fwd_zb = nullptr, colz_conv_zb = nullptr;  // N >= 64
   hipFunction_t xy1_fwd[cfgeo::kSplitVariants] = {}, xy1_inv[cfgeo::kSplitVariants] = {};  // N = 256
@@ -295,6 +296,16 @@ int size_res(unsigned n, SizeFns** out) {
       CFCHK(get_fn(t.f, name));
     }
   }
+  if (cfgeo::cube_supported((int)n)) {
+    struct {
+      hipFunction_t* f;
+      const char* fmt;
+    } cu[] = {{&s.cube_fwd, "cf_cube_fwd_%u"}, {&s.cube_inv, "cf_cube_inv_%u"}, {&s.cube_conv, "cf_cube_conv_%u"}};
+    for (auto& t : cu) {
+      snprintf(name, sizeof name, t.fmt, n);
+      CFCHK(get_fn(t.f, name));
+    }
+  }
   if (cfgeo::plane_supported((int)n)) {
     snprintf(name, sizeof name, "cf_plane_fwd_%u", n);
     CFCHK(get_fn(&s.plane_fwd, name));
@@ -416,9 +427,13 @@ int launch_pass(const Pass& p, unsigned n, unsigned nb, hipStream_t s, const voi
   return CF_OK;
 }
 
-// forward 3D FFT: x, y, z passes (in may equal out)
+// forward 3D FFT: x, y, z passes, or one pass over whole cubes (in may equal out)
 void fwd_passes(const SizeFns& f, unsigned n, unsigned nb, const void* in, void* out, PassList& v) {
   const double io = 2.0 * cube_bytes(n) * nb;
+  if (cfgeo::cube_supported((int)n)) {
+    v.push_back({f.cube_fwd, 1, n * n, in, out, nullptr, 0, 1.0f, "xyz_fwd", io});
+    return;
+  }
   const unsigned rt = cfgeo::row_threads(n), rT = cfgeo::row_tiles(n);
   const unsigned ct = cfgeo::col_threads(n), cT = cfgeo::col_tiles(n);
   v.push_back({f.row_fwd, rT, rt, in, out, nullptr, 0, 1.0f, "x_fwd", io});
@@ -428,6 +443,10 @@ void fwd_passes(const SizeFns& f, unsigned n, unsigned nb, const void* in, void*
 
 void inv_passes(const SizeFns& f, unsigned n, unsigned nb, const void* in, void* out, float scale, PassList& v) {
   const double io = 2.0 * cube_bytes(n) * nb;
+  if (cfgeo::cube_supported((int)n)) {
+    v.push_back({f.cube_inv, 1, n * n, in, out, nullptr, 0, scale, "xyz_inv", io});
+    return;
+  }
   const unsigned rt = cfgeo::row_threads(n), rT = cfgeo::row_tiles(n);
   const unsigned ct = cfgeo::col_threads(n), cT = cfgeo::col_tiles(n);
   v.push_back({f.colz_inv, cT, ct, in, out, nullptr, 0, 1.0f, "z_inv", io});
@@ -438,10 +457,12 @@ void inv_passes(const SizeFns& f, unsigned n, unsigned nb, const void* in, void*
 // Convolution passes of `plan`.  AXIS5: x, y, z*H*z, y^-1, x^-1(+scale), in
 // place in out.  PLANE3: xy-plane, z*H*z, xy-plane^-1(+scale), in place.
 // SPLIT3: sig -> work (pass A), work in place (middle), work -> out (pass C).
+// AXIS5 at N = 8 and 16: one pass over whole cubes, unless the caller reports
+// the forward and the inverse half separately (same bits either way).
 // Returns the index of the first pass after the product (the fpga_t split).
 size_t conv_passes(const SizeFns& f, int plan, unsigned n, unsigned nb, const void* sig, void* out, void* work,
                    const void* H, long long hstride, float scale, PassList& v,
-                   int precision = CF_PREC_FP32) {
+                   int precision = CF_PREC_FP32, bool separate_inverse = false) {
   const double V = (double)cube_bytes(n);
   const double io = 2.0 * V * nb;
   const double hbytes = hstride ? V * nb : V;
@@ -509,6 +530,10 @@ size_t conv_passes(const SizeFns& f, int plan, unsigned n, unsigned nb, const vo
     v.push_back({f.coly_inv_zb, cT, ct, work, out, nullptr, 0, 1.0f, "y_inv", io});
     v.push_back({f.row_inv, rT, rt, out, out, nullptr, 0, scale, "x_inv", io});
     return split;
+  }
+  if (cfgeo::cube_supported((int)n) && !separate_inverse) {
+    v.push_back({f.cube_conv, 1, n * n, sig, out, H, hstride, scale, "xyz_fwd_mul_inv", io + hbytes});
+    return v.size();
   }
   v.push_back({f.row_fwd, rT, rt, sig, out, nullptr, 0, 1.0f, "x_fwd", io});
   v.push_back({f.coly_fwd, cT, ct, out, out, nullptr, 0, 1.0f, "y_fwd", io});
@@ -1278,7 +1303,8 @@ extern "C" int cfe_conv_host(unsigned n, const void* sig, const void* filter, vo
     CFCHK(staged_h2d(g.d_data, sig, SV, s));
     HIPCHK(hipStreamSynchronize(s));
     auto t3 = clk::now();
-    const size_t split = conv_passes(*f, plan, n, how_many, g.d_data, g.d_data, work, g.d_filt, 0, 1.0f, conv_p);
+    const size_t split = conv_passes(*f, plan, n, how_many, g.d_data, g.d_data, work, g.d_filt, 0, 1.0f, conv_p,
+                                     CF_PREC_FP32, true);
     const size_t nc = conv_p.size();
     hipEvent_t* ec = ev + 1 + nf;
     CFCHK(run_passes(conv_p, n, how_many, s, f->tw, ec));  // ec[0 .. nc]
@@ -1306,7 +1332,8 @@ extern "C" int cfe_conv_host(unsigned n, const void* sig, const void* filter, vo
   spectrum_passes(*f, plan, n, 1, mapped(g.h_filt), g.d_filt, work, filt_p);
   const size_t nf = filt_p.size();
   CFCHK(run_passes(filt_p, n, 1, s, f->tw, ev));  // ev[0 .. nf]
-  const size_t split = conv_passes(*f, plan, n, how_many, mapped(g.h_sig), g.d_data, work, g.d_filt, 0, 1.0f, conv_p);
+  const size_t split = conv_passes(*f, plan, n, how_many, mapped(g.h_sig), g.d_data, work, g.d_filt, 0, 1.0f, conv_p,
+                                     CF_PREC_FP32, true);
   conv_p.back().out = mapped(g.h_out);  // the last pass writes host memory directly
   const size_t nc = conv_p.size();
   hipEvent_t* ec = ev + nf + 1;

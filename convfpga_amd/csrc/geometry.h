@@ -27,6 +27,9 @@ constexpr int row_tiles(int n) { return n * n / row_l(n); }
 
 constexpr bool supported(int n) { return points_per_thread(n) != 0; }
 
+// a whole cube per work-group, one line of n points per thread (n*n threads)
+constexpr bool cube_supported(int n) { return n == 8 || n == 16; }
+
 // 3-pass plane schedule (N <= 128): one xy-plane per work-group
 constexpr bool plane_supported(int n) { return n == 32 || n == 64 || n == 128; }
 constexpr int plane_threads(int n) { return n * threads_per_line(n); }

@@ -13,6 +13,7 @@
 #include "axis_passes.h"
 #include "batch_kernel.h"
 #include "fft_core.h"
+#include "small_cube.h"
 #include "three_pass.h"
 #include "split_mfma.h"
 #include "split_mfma512.h"
@@ -82,6 +83,21 @@ CF_INSTANTIATE_ZB(64)
 CF_INSTANTIATE_ZB(128)
 CF_INSTANTIATE_ZB(256)
 CF_INSTANTIATE_ZB(512)
+
+// ---- whole cubes of edge 8 and 16 (small_cube.h): ntotal cubes, one work-group each ------
+#define CF_CUBE(N)                                                                                             \
+  static_assert(cfgeo::cube_supported(N), "cube geometry");                                                    \
+  extern "C" __global__ __launch_bounds__(cfk::CubeCfg<N>::THREADS) void cf_cube_fwd_##N(CF_ARGS) {             \
+    cfk::cube_kernel<N, 0>(in, out, H, hstride, scale, ntotal);                                                \
+  }                                                                                                            \
+  extern "C" __global__ __launch_bounds__(cfk::CubeCfg<N>::THREADS) void cf_cube_inv_##N(CF_ARGS) {             \
+    cfk::cube_kernel<N, 1>(in, out, H, hstride, scale, ntotal);                                                \
+  }                                                                                                            \
+  extern "C" __global__ __launch_bounds__(cfk::CubeCfg<N>::THREADS) void cf_cube_conv_##N(CF_ARGS) {            \
+    cfk::cube_kernel<N, 2>(in, out, H, hstride, scale, ntotal);                                                \
+  }
+CF_CUBE(8)
+CF_CUBE(16)
 
 // ---- 3-pass schedules (three_pass.h) ------------------------------------------
 #define CF_PLANE(N)                                                                                   \
