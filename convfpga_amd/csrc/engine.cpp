@@ -599,6 +599,37 @@ int run_passes(const PassList& v, unsigned n, unsigned nb, hipStream_t s, const 
   return CF_OK;
 }
 
+// How many of `count` cubes of edge n go through a schedule's passes together:
+// groups of about kGroupBytes of cubes, evenly sized.  The next pass then finds
+// what a pass wrote in the 256 MiB memory-side cache.  Passes over the whole
+// batch against groups (us per call; one group when the batch holds fewer than
+// two of them): 4 x 256^3 own filters 752 -> 648, split-FP16 920 -> 812; 40 x
+// 128^3 824 -> 786 in groups of 8 (854 in groups of 4, whose passes no longer
+// fill the GPU; 822 in groups of 10); 300 x 64^3 721 -> 637 in groups of 64
+// (783 of 16); 4 transforms of 256^3 651 -> 535.
+constexpr size_t kGroupBytes = size_t(128) << 20;
+unsigned pass_group(unsigned n, unsigned count) {
+  const unsigned per = (unsigned)std::max<size_t>(1, kGroupBytes / cube_bytes(n));
+  const unsigned groups = std::max(1u, count / per);
+  return count / groups + (count % groups != 0);
+}
+
+// The convolution passes over how_many cubes, group by group.  work holds the
+// intermediates of one group (work_bytes of pass_group(n, how_many) cubes).
+int run_conv(const SizeFns& f, int plan, unsigned n, unsigned how_many, const void* sig, void* out, void* work,
+             const void* H, long long hstride, float scale, int precision, hipStream_t s) {
+  const unsigned group = pass_group(n, how_many);
+  const size_t V = cube_bytes(n);
+  for (unsigned b = 0; b < how_many; b += group) {
+    const unsigned nb = std::min(group, how_many - b);
+    PassList p;
+    conv_passes(f, plan, n, nb, (const char*)sig + b * V, (char*)out + b * V, work,
+                (const char*)H + (size_t)b * hstride * 8, hstride, scale, p, precision);
+    CFCHK(run_passes(p, n, nb, s, f.tw, nullptr));
+  }
+  return CF_OK;
+}
+
 int ensure_device(void** p, size_t* have, size_t need) {
   if (*have >= need) return CF_OK;
   if (*p) (void)hipFree(*p);
@@ -1395,13 +1426,15 @@ extern "C" int cf_spectrum_create(unsigned n, unsigned count, const void* filter
   int rc = e == hipSuccess ? choose_plan(n, f, &h->plan)
                            : fail(CF_ERR_RUNTIME, "hipMemcpyAsync: %s", hipGetErrorString(e));
   void* work = nullptr;
-  if (rc == CF_OK && needs_work(h->plan)) rc = acquire_work(bytes, s, &work);
-  if (rc == CF_OK) {
+  const unsigned group = pass_group(n, count);
+  if (rc == CF_OK && needs_work(h->plan)) rc = acquire_work(cube_bytes(n) * group, s, &work);
+  for (unsigned b = 0; b < count && rc == CF_OK; b += group) {
+    const unsigned nb = std::min(group, count - b);
     PassList p;
-    spectrum_passes(*f, h->plan, n, count, src, h->d, work, p);
-    rc = run_passes(p, n, count, s, f->tw, nullptr);
-    if (rc == CF_OK && work) rc = release_work(s);
+    spectrum_passes(*f, h->plan, n, nb, (const char*)src + b * cube_bytes(n), (char*)h->d + b * cube_bytes(n), work, p);
+    rc = run_passes(p, n, nb, s, f->tw, nullptr);
   }
+  if (work) release_work(s);
   if (rc == CF_OK && hipStreamSynchronize(s) != hipSuccess) rc = fail(CF_ERR_RUNTIME, "spectrum setup failed");
   if (rc != CF_OK) {
     (void)hipFree(h->d);
@@ -1502,10 +1535,13 @@ static int conv_device_impl(cf_spectrum_t h, const void* d_sig, void* d_out, uns
   const float scale = scale_mode == CF_SCALE_INV_N3 ? (float)(1.0 / (double)cube_elems(n)) : 1.0f;
   const long long hstride = h->count == 1 ? 0 : (long long)cube_elems(n);
   hipStream_t s = (hipStream_t)stream;
+  // armed by cf_profile_begin: the last call of every group of prof_every (a
+  // call that follows others in the stream, not one that starts from an idle GPU)
+  const bool profiled = !times && g.prof_max > g.prof_calls && ++g.prof_seen % g.prof_every == 0;
+  // a call whose passes are timed runs each of them over the whole batch
+  const unsigned group = times || profiled ? how_many : pass_group(n, how_many);
   void* work = nullptr;
-  if (needs_work(h->plan)) CFCHK(acquire_work(work_bytes(h->plan, n, how_many, d_sig, d_out), s, &work));
-  PassList p;
-  conv_passes(*f, h->plan, n, how_many, d_sig, d_out, work, h->d, hstride, scale, p, precision);
+  if (needs_work(h->plan)) CFCHK(acquire_work(work_bytes(h->plan, n, group, d_sig, d_out), s, &work));
   struct WorkRelease {  // the workspace is marked busy on s whatever path returns
     void* w;
     hipStream_t s;
@@ -1513,25 +1549,24 @@ static int conv_device_impl(cf_spectrum_t h, const void* d_sig, void* d_out, uns
       if (w) release_work(s);
     }
   } wr{work, s};
-  if (!times) {
-    // armed by cf_profile_begin: the last call of every group of prof_every (a
-    // call that follows others in the stream, not one that starts from an idle GPU)
-    if (g.prof_max > g.prof_calls && ++g.prof_seen % g.prof_every == 0) {
-      hipEvent_t* ev = &g.prof_ev[(size_t)g.prof_calls * (CF_MAX_PASSES + 1)];
-      CFCHK(run_passes(p, n, how_many, s, f->tw, ev));
-      if (g.prof_calls == 0) {
-        g.prof_npass = (unsigned)p.size();
-        g.prof_names.clear();
-        g.prof_bytes.clear();
-        for (auto& q : p) {
-          g.prof_names.push_back(q.name);
-          g.prof_bytes.push_back(q.bytes);
-        }
+  if (!times && !profiled)
+    return run_conv(*f, h->plan, n, how_many, d_sig, d_out, work, h->d, hstride, scale, precision, s);
+  PassList p;
+  conv_passes(*f, h->plan, n, how_many, d_sig, d_out, work, h->d, hstride, scale, p, precision);
+  if (profiled) {
+    hipEvent_t* ev = &g.prof_ev[(size_t)g.prof_calls * (CF_MAX_PASSES + 1)];
+    CFCHK(run_passes(p, n, how_many, s, f->tw, ev));
+    if (g.prof_calls == 0) {
+      g.prof_npass = (unsigned)p.size();
+      g.prof_names.clear();
+      g.prof_bytes.clear();
+      for (auto& q : p) {
+        g.prof_names.push_back(q.name);
+        g.prof_bytes.push_back(q.bytes);
       }
-      ++g.prof_calls;
-      return CF_OK;
     }
-    return run_passes(p, n, how_many, s, f->tw, nullptr);
+    ++g.prof_calls;
+    return CF_OK;
   }
   CFCHK(ensure_events());
   CFCHK(run_passes(p, n, how_many, s, f->tw, g.ev));
@@ -1580,9 +1615,7 @@ extern "C" int cf_conv3d_device_noalloc(cf_spectrum_t h, const void* d_sig, void
   }
   const float scale = scale_mode == CF_SCALE_INV_N3 ? (float)(1.0 / (double)cube_elems(n)) : 1.0f;
   const long long hstride = h->count == 1 ? 0 : (long long)cube_elems(n);
-  PassList p;
-  conv_passes(f, h->plan, n, how_many, d_sig, d_out, work, h->d, hstride, scale, p, precision);
-  return run_passes(p, n, how_many, (hipStream_t)stream, f.tw, nullptr);
+  return run_conv(f, h->plan, n, how_many, d_sig, d_out, work, h->d, hstride, scale, precision, (hipStream_t)stream);
 }
 
 extern "C" int cf_conv3d_host(cf_spectrum_t h, const void* h_sig, void* h_out, unsigned how_many, int scale_mode,
@@ -1721,12 +1754,19 @@ extern "C" int cf_fft3d_device(unsigned n, const void* d_in, void* d_out, unsign
   CFCHK(require_ready());
   SizeFns* f = nullptr;
   CFCHK(size_res(n, &f));
-  PassList p;
-  if (inverse)
-    inv_passes(*f, n, how_many, d_in, d_out, 1.0f, p);
-  else
-    fwd_passes(*f, n, how_many, d_in, d_out, p);
-  return run_passes(p, n, how_many, (hipStream_t)stream, f->tw, nullptr);
+  const unsigned group = pass_group(n, how_many);
+  for (unsigned b = 0; b < how_many; b += group) {
+    const unsigned nb = std::min(group, how_many - b);
+    const void* in = (const char*)d_in + b * cube_bytes(n);
+    void* out = (char*)d_out + b * cube_bytes(n);
+    PassList p;
+    if (inverse)
+      inv_passes(*f, n, nb, in, out, 1.0f, p);
+    else
+      fwd_passes(*f, n, nb, in, out, p);
+    CFCHK(run_passes(p, n, nb, (hipStream_t)stream, f->tw, nullptr));
+  }
+  return CF_OK;
 }
 
 extern "C" int cf_rel_l2_device(const void* d_test, const void* d_ref, int ref_is_f64, size_t npts, void* stream,
@@ -2121,7 +2161,8 @@ static int batch_create(const cf_instance_t* inst, unsigned count, int scale_mod
              (const char*)inst[i + run].d_sig == (const char*)inst[i].d_sig + run * V &&
              (char*)inst[i + run].d_out == (char*)inst[i].d_out + run * V)
         ++run;
-      work_need = std::max(work_need, work_bytes(inst[i].h->plan, n, run, inst[i].d_sig, inst[i].d_out));
+      work_need = std::max(work_need, work_bytes(inst[i].h->plan, n, pass_group(n, run), inst[i].d_sig,
+                                                 inst[i].d_out));
       runs.push_back({i, run, shared});
       i += run;
     }
@@ -2138,10 +2179,8 @@ static int batch_create(const cf_instance_t* inst, unsigned count, int scale_mod
       const unsigned i = r.i, n = inst[i].h->n;
       const long long hstride = (r.run > 1 && !r.shared) ? (long long)cube_elems(n) : 0;
       const float scale = scale_mode == CF_SCALE_INV_N3 ? (float)(1.0 / (double)cube_elems(n)) : 1.0f;
-      PassList p;
-      conv_passes(*fns[i], inst[i].h->plan, n, r.run, inst[i].d_sig, inst[i].d_out, b->d_work, inst[i].h->d, hstride,
-                  scale, p);
-      rc = run_passes(p, n, r.run, g.capture, fns[i]->tw, nullptr);
+      rc = run_conv(*fns[i], inst[i].h->plan, n, r.run, inst[i].d_sig, inst[i].d_out, b->d_work, inst[i].h->d, hstride,
+                    scale, CF_PREC_FP32, g.capture);
     }
     rc = batch_capture_end(b, rc);
   }

@@ -1,0 +1,48 @@
+"""Batches whose cubes go through the passes in groups (pass_group, engine.cpp):
+each cube's result is, bit for bit, that of a call on the cube alone, whatever
+the group it falls in, for counts around the points where the grouping changes."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _same(a, b):
+    import torch
+    torch.cuda.synchronize()
+    return torch.equal(torch.view_as_real(a).view(torch.int32), torch.view_as_real(b).view(torch.int32))
+
+
+# 128 MiB of cubes make a group: 8 at 128^3, 64 at 64^3, 1 at 256^3
+@pytest.mark.parametrize("n,count", [(128, 15), (128, 17), (64, 130), (256, 2), (256, 3)])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_groups_equal_single_cubes(gpu, n, count, in_place):
+    import torch
+    api = gpu.api
+    print("case groups N=%d count=%d in_place=%s" % (n, count, in_place), flush=True)
+    P = n ** 3
+    sig = torch.empty((count, P), dtype=torch.complex64, device="cuda")
+    filt = torch.empty_like(sig)
+    api.fill_uniform(sig, 2 * sig.numel(), 61000 + n + count)
+    api.fill_uniform(filt, 2 * filt.numel(), 62000 + n + count)
+    own, shared = gpu.Spectrum(n, filt, count), gpu.Spectrum(n, filt)
+    tr = torch.empty_like(sig)
+    gpu.fft3d_device(n, sig, tr, count, inverse=in_place)
+    out, out_sh = (sig.clone(), sig.clone()) if in_place else (torch.empty_like(sig), torch.empty_like(sig))
+    gpu.conv3d_device(own, out if in_place else sig, out, count)
+    gpu.conv3d_device(shared, out_sh if in_place else sig, out_sh, count)
+    batch_out = torch.empty_like(sig)
+    views = [own.view(k) for k in range(count)]
+    batch = api.Batch([(sig[k], batch_out[k], views[k]) for k in range(count)], mode=api.CF_BATCH_GRAPH)
+    batch.launch()
+    batch.check()
+    one = torch.empty_like(sig[0])
+    for k in range(count):
+        alone = gpu.Spectrum(n, filt[k])
+        gpu.conv3d_device(alone, sig[k], one)
+        assert _same(one, out[k]) and _same(one, batch_out[k]), k
+        gpu.conv3d_device(shared, sig[k], one)
+        assert _same(one, out_sh[k]), k
+        gpu.fft3d_device(n, sig[k], one, inverse=in_place)
+        assert _same(one, tr[k]), k
+        alone.close()
+    batch.close()
