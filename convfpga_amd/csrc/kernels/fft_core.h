@@ -299,6 +299,55 @@ __device__ __forceinline__ void fft_line(float2 (&v)[Shape<N>::P], int t, const 
   if constexpr (NS >= 3) fft_step<N, S::R2, S::R0 * S::R1, true, INV, WAVE>(v, t, lds, tw);
 }
 
+// The same with the exchange moved in halves, real parts then imaginary parts,
+// through a float view: half the LDS for two more synchronisations per step.
+template <int N, int R, int NSP, bool LAST, bool INV, bool WAVE, class LdsF>
+__device__ __forceinline__ void fft_step_half(float2 (&v)[Shape<N>::P], int t, const LdsF& lds, const float2* tw) {
+  constexpr int P = Shape<N>::P, T = N / P, Q = P / R;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int k = (t + T * q) & (NSP - 1);
+    float2 u[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) u[r] = v[q + r * Q];
+    if constexpr (NSP > 1) {
+#pragma unroll
+      for (int r = 1; r < R; ++r) u[r] = cmulw<INV>(u[r], tw[r * k * (N / (NSP * R))]);
+    }
+    DFT<R, INV>::run(u);
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[q + r * Q] = u[r];
+  }
+  if constexpr (!LAST) {
+    auto put = [&](auto part) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const int vv = t + T * q, k = vv & (NSP - 1), base = (vv - k) * R + k;
+#pragma unroll
+        for (int r = 0; r < R; ++r) lds.st(base + r * NSP, part(v[q + r * Q]));
+      }
+      lds_sync<WAVE>();
+    };
+    put([](const float2& x) { return x.x; });
+    float re[P];
+#pragma unroll
+    for (int m = 0; m < P; ++m) re[m] = lds.ld(t + T * m);
+    lds_sync<WAVE>();
+    put([](const float2& x) { return x.y; });
+#pragma unroll
+    for (int m = 0; m < P; ++m) v[m] = make_float2(re[m], lds.ld(t + T * m));
+    lds_sync<WAVE>();
+  }
+}
+template <int N, bool INV, bool WAVE = false, class LdsF>
+__device__ __forceinline__ void fft_line_half(float2 (&v)[Shape<N>::P], int t, const LdsF& lds, const float2* tw) {
+  using S = Shape<N>;
+  constexpr int NS = ShapeInfo<N>::NSTEPS;
+  fft_step_half<N, S::R0, 1, NS == 1, INV, WAVE>(v, t, lds, tw);
+  if constexpr (NS >= 2) fft_step_half<N, S::R1, S::R0, NS == 2, INV, WAVE>(v, t, lds, tw);
+  if constexpr (NS >= 3) fft_step_half<N, S::R2, S::R0 * S::R1, true, INV, WAVE>(v, t, lds, tw);
+}
+
 // LDS views.  Column layout (lines are adjacent x-columns, C per tile):
 // element (point o, column c) at o*(C+1) + c -- the +1 pad staggers rows by
 // one bank pair.  Row layout (lines are contiguous x-rows): point o at
@@ -320,6 +369,19 @@ struct RowLds {
   float2* p;  // start of this row's segment
   __device__ __forceinline__ void st(int o, float2 x) const { p[o + (o >> 4)] = x; }
   __device__ __forceinline__ float2 ld(int o) const { return p[o + (o >> 4)]; }
+};
+
+// float views of the half-width exchanges: a row's segment, a column of pitch PITCH
+struct RowLdsF {
+  float* p;
+  __device__ __forceinline__ void st(int o, float x) const { p[o + (o >> 4)] = x; }
+  __device__ __forceinline__ float ld(int o) const { return p[o + (o >> 4)]; }
+};
+template <int PITCH>
+struct ColLdsF {
+  float* p;
+  __device__ __forceinline__ void st(int o, float x) const { p[o * PITCH] = x; }
+  __device__ __forceinline__ float ld(int o) const { return p[o * PITCH]; }
 };
 
 template <int N, int THREADS>

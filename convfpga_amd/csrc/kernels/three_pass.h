@@ -39,6 +39,16 @@ struct PlaneCfg {
   static constexpr int ROW_PITCH = N + N / 16;
   static constexpr int COL_PITCH = N + 1;
   static constexpr int LDS = N * (ROW_PITCH > COL_PITCH ? ROW_PITCH : COL_PITCH);
+  // A 128 x 128 plane (1024 threads) would fill a CU's LDS by itself (137 KiB):
+  // its exchanges move real parts, then imaginary parts, through one float
+  // array (68 KiB), so that two work-groups share a CU and one computes while
+  // the other loads or stores.  Planes of 3 / 16 cubes forward: 31 / 135 -> 25 /
+  // 113 us (events included), of one cube (128 work-groups) the same.
+  static constexpr bool HALF = N == 128;
+  // float rows of the half-width exchange: 136 = 8 (mod 64), so that the 8 rows
+  // by 8 points of a wave's row accesses fall on 64 different banks
+  static constexpr int H_PITCH = N + 8;
+  static constexpr int H_LDS = N * H_PITCH / 2;  // in float2
 };
 
 // Column view of the plane buffer: (point y, column kx) at y*(N+1) + kx.
@@ -76,9 +86,46 @@ struct PlanePass {
       for (int m = 0; m < P; ++m) r.v[m] = src[(ct + T * m) * N + ck];
     }
   }
+  // rows <-> columns through the float array, real then imaginary parts
+  template <bool TO_COLS>
+  __device__ __forceinline__ void turn_half(Regs& r, float* f) const {
+    float* const rowp = f + ry * K::H_PITCH + rt;   // x = rt + T*m
+    float* const colp = f + ct * K::H_PITCH + ck;   // y = ct + T*m
+    constexpr int CS = T * K::H_PITCH;
+    float re[P];
+#pragma unroll
+    for (int m = 0; m < P; ++m) *(TO_COLS ? rowp + T * m : colp + CS * m) = r.v[m].x;
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < P; ++m) re[m] = *(TO_COLS ? colp + CS * m : rowp + T * m);
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < P; ++m) *(TO_COLS ? rowp + T * m : colp + CS * m) = r.v[m].y;
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < P; ++m) r.v[m] = make_float2(re[m], *(TO_COLS ? colp + CS * m : rowp + T * m));
+    __syncthreads();
+  }
   __device__ __forceinline__ void process(int tile, Regs& r) const {
     float2* dst = out + (size_t)tile * N * N;
-    if constexpr (!INV) {
+    if constexpr (K::HALF) {
+      float* const f = reinterpret_cast<float*>(lds);
+      const RowLdsF row{f + ry * K::H_PITCH};  // N + N/16 <= H_PITCH floats
+      const ColLdsF<K::H_PITCH> col{f + ck};
+      if constexpr (!INV) {
+        fft_line_half<N, false, true>(r.v, rt, row, tw_s);  // a row: lanes of one wave
+        turn_half<true>(r, f);  // (it first rewrites each wave's own rows)
+        fft_line_half<N, false>(r.v, ct, col, tw_s);
+#pragma unroll
+        for (int m = 0; m < P; ++m) dst[(ct + T * m) * N + ck] = r.v[m];
+      } else {
+        fft_line_half<N, true>(r.v, ct, col, tw_s);
+        turn_half<false>(r, f);
+        fft_line_half<N, true, true>(r.v, rt, row, tw_s);
+#pragma unroll
+        for (int m = 0; m < P; ++m) dst[ry * N + rt + T * m] = cscale(r.v[m], scale);
+      }
+    } else if constexpr (!INV) {
       fft_line<N, false, true>(r.v, rt, RowLds{lds + ry * K::ROW_PITCH}, tw_s);  // a row: lanes of one wave
       __syncthreads();  // every wave has read its rows before the transpose overwrites them
 #pragma unroll
@@ -108,7 +155,7 @@ struct PlanePass {
 template <int N, bool INV>
 __device__ __forceinline__ void plane_kernel(const float2* in, float2* out, const float2* tw, float scale, int ntotal) {
   using K = PlaneCfg<N>;
-  __shared__ float2 lds[K::LDS];
+  __shared__ float2 lds[K::HALF ? K::H_LDS : K::LDS];
   __shared__ float2 tw_s[N];
   const int x = threadIdx.x;
   const PlanePass<N, INV> k{in, out, tw_s, lds, scale, x % K::T, x / K::T, x % N, x / N};
