@@ -70,6 +70,7 @@ struct SizeFns {
   hipFunction_t coly_fwd_zb = nullptr, coly_inv_zb = nullptr, colz_fwd_zb = nullptr, colz_conv_zb = nullptr;  // N >= 64
   hipFunction_t xy1_fwd[cfgeo::kSplitVariants] = {}, xy1_inv[cfgeo::kSplitVariants] = {};  // N = 256
   hipFunction_t mid[cfgeo::kSplitVariants] = {}, mspec[cfgeo::kSplitVariants] = {};
+  hipFunction_t fft2_first[2] = {}, fft2_second[2] = {};  // N = 256, plain transform: forward, inverse
   hipFunction_t mx_xy1_fwd = nullptr, mx_xy1_inv = nullptr, mx_mid = nullptr;  // N = 256, split-FP16 MFMA
   // N = 512, split-FP16 MFMA axis passes: natural layout, then z-blocked (AXIS5Z)
   hipFunction_t mx_row_fwd = nullptr, mx_row_inv = nullptr, mx_coly_fwd = nullptr, mx_coly_inv = nullptr;
@@ -107,6 +108,15 @@ bool plan_ok(unsigned n, int plan) {
   return false;
 }
 
+// Device workspace shared by the calls of all streams, ordered by ev.
+struct Workspace {
+  void* d = nullptr;
+  size_t bytes = 0;
+  hipStream_t stream = nullptr;  // of the last user
+  bool used = false;
+  hipEvent_t ev = nullptr;
+};
+
 struct Engine {
   std::recursive_mutex mu;
   bool ready = false;
@@ -134,12 +144,10 @@ struct Engine {
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
   bool stage_used[2] = {false, false};
   size_t h_out_bytes = 0;
-  // workspace of the 3-pass four-step plans, ordered across streams by work_ev
-  void* d_work = nullptr;
-  size_t d_work_bytes = 0;
-  hipStream_t work_stream = nullptr;
-  bool work_used = false;
-  hipEvent_t work_ev = nullptr;
+  Workspace work;      // of the plans that go through one
+  Workspace fft_work;  // of the two-pass plain transform; of its own, so that a transform
+                       // meets neither the convolutions of other streams nor a graph
+                       // that holds the address of theirs
   std::string arch;
   // error-norm scratch
   void* d_err = nullptr;
@@ -149,9 +157,10 @@ struct Engine {
   // only device this engine drives), looked up once when the module is loaded
   void* scratch = nullptr;
   size_t scratch_bytes = 0;
-  // cf_profile_begin/end: events of up to prof_max calls, (CF_MAX_PASSES+1) each
+  // cf_profile_begin/end: sets of CF_MAX_PASSES+1 events, at least one for each of up to prof_max calls
   std::vector<hipEvent_t> prof_ev;
   unsigned prof_max = 0, prof_calls = 0, prof_npass = 0;
+  size_t prof_sets = 0;  // sets of events recorded: one per group of cubes of each recorded call
   unsigned prof_every = 1, prof_seen = 0;  // record the last call of every group of prof_every while armed
   std::vector<std::string> prof_names;
   std::vector<double> prof_bytes;
@@ -182,13 +191,11 @@ void release_all() {
   if (g.d_data) (void)hipFree(g.d_data);
   if (g.d_filt) (void)hipFree(g.d_filt);
   if (g.d_err) (void)hipFree(g.d_err);
-  if (g.d_work) (void)hipFree(g.d_work);
-  g.d_work = nullptr;
-  g.d_work_bytes = 0;
-  g.work_used = false;
-  g.work_stream = nullptr;
-  if (g.work_ev) (void)hipEventDestroy(g.work_ev);
-  g.work_ev = nullptr;
+  for (Workspace* w : {&g.work, &g.fft_work}) {
+    if (w->d) (void)hipFree(w->d);
+    if (w->ev) (void)hipEventDestroy(w->ev);
+    *w = Workspace();
+  }
   if (g.h_sig) (void)hipHostFree(g.h_sig);
   if (g.h_filt) (void)hipHostFree(g.h_filt);
   if (g.h_out) (void)hipHostFree(g.h_out);
@@ -209,6 +216,7 @@ void release_all() {
   for (auto e : g.prof_ev) (void)hipEventDestroy(e);
   g.prof_ev.clear();
   g.prof_max = g.prof_calls = 0;
+  g.prof_sets = 0;
   if (g.stream) (void)hipStreamDestroy(g.stream);
   g.stream = nullptr;
   if (g.mod) (void)hipModuleUnload(g.mod);
@@ -343,6 +351,10 @@ int size_res(unsigned n, SizeFns** out) {
     CFCHK(get_fn(&s.mspec[vi], name));
   }
   if (n == 256) {
+    CFCHK(get_fn(&s.fft2_first[0], "cf_fft2_first_fwd_256"));
+    CFCHK(get_fn(&s.fft2_first[1], "cf_fft2_first_inv_256"));
+    CFCHK(get_fn(&s.fft2_second[0], "cf_fft2_second_fwd_256"));
+    CFCHK(get_fn(&s.fft2_second[1], "cf_fft2_second_inv_256"));
     CFCHK(get_fn(&s.mx_xy1_fwd, "cf_xy1_fwd_256_s24"));
     CFCHK(get_fn(&s.mx_xy1_inv, "cf_xy1_inv_256_s24"));
     CFCHK(get_fn(&s.mx_mid, "cf_mid_256_s24m2"));
@@ -752,44 +764,46 @@ double host_ms(std::chrono::steady_clock::time_point a, std::chrono::steady_cloc
 }
 
 // Workspace of `bytes` for a call on stream s.  Calls on different streams are
-// ordered through work_ev so that they never overlap on the shared workspace.
-int acquire_work(size_t bytes, hipStream_t s, void** out) {
-  if (!g.work_ev) HIPCHK(hipEventCreateWithFlags(&g.work_ev, hipEventDisableTiming));
-  if (g.d_work_bytes < bytes) {
-    if (g.d_work) {
+// ordered through w.ev so that they never overlap on it.
+int acquire_work(Workspace& w, size_t bytes, hipStream_t s, void** out) {
+  if (!w.ev) HIPCHK(hipEventCreateWithFlags(&w.ev, hipEventDisableTiming));
+  if (w.bytes < bytes) {
+    if (w.d) {
       HIPCHK(hipDeviceSynchronize());  // earlier users on any stream are done
-      (void)hipFree(g.d_work);
+      (void)hipFree(w.d);
     }
-    g.d_work = nullptr;
-    g.d_work_bytes = 0;
-    g.work_used = false;
-    hipError_t e = hipMalloc(&g.d_work, bytes);
+    w.d = nullptr;
+    w.bytes = 0;
+    w.used = false;
+    hipError_t e = hipMalloc(&w.d, bytes);
     if (e != hipSuccess) return fail(CF_ERR_NOMEM, "hipMalloc(%zu) for the workspace: %s", bytes, hipGetErrorString(e));
-    g.d_work_bytes = bytes;
+    w.bytes = bytes;
   }
-  if (g.work_used && g.work_stream != s) {
+  if (w.used && w.stream != s) {
     // Everything submitted so far to the previous user's stream includes its
     // use of the workspace, so an event recorded there now orders s after it.
     // (Recording lazily, only on a change of stream, keeps event packets --
     // each a gap of several microseconds on the GPU -- out of the
     // single-stream sequence.)  A stream destroyed meanwhile has finished its
     // work; should the record fail, wait for the whole device instead.
-    if (hipEventRecord(g.work_ev, g.work_stream) == hipSuccess) {
-      HIPCHK(hipStreamWaitEvent(s, g.work_ev, 0));
+    if (hipEventRecord(w.ev, w.stream) == hipSuccess) {
+      HIPCHK(hipStreamWaitEvent(s, w.ev, 0));
     } else {
       (void)hipGetLastError();
       HIPCHK(hipDeviceSynchronize());
     }
   }
-  *out = g.d_work;
+  *out = w.d;
   return CF_OK;
 }
+int acquire_work(size_t bytes, hipStream_t s, void** out) { return acquire_work(g.work, bytes, s, out); }
 
-int release_work(hipStream_t s) {
-  g.work_stream = s;
-  g.work_used = true;
+int release_work(Workspace& w, hipStream_t s) {
+  w.stream = s;
+  w.used = true;
   return CF_OK;
 }
+int release_work(hipStream_t s) { return release_work(g.work, s); }
 
 int ensure_events() {
   for (auto& e : g.ev)
@@ -1542,11 +1556,7 @@ static int conv_device_impl(cf_spectrum_t h, const void* d_sig, void* d_out, uns
   const float scale = scale_mode == CF_SCALE_INV_N3 ? (float)(1.0 / (double)cube_elems(n)) : 1.0f;
   const long long hstride = h->count == 1 ? 0 : (long long)cube_elems(n);
   hipStream_t s = (hipStream_t)stream;
-  // armed by cf_profile_begin: the last call of every group of prof_every (a
-  // call that follows others in the stream, not one that starts from an idle GPU)
-  const bool profiled = !times && g.prof_max > g.prof_calls && ++g.prof_seen % g.prof_every == 0;
-  // a call whose passes are timed runs each of them over the whole batch
-  const unsigned group = times || profiled ? how_many : pass_group(n, how_many);
+  const unsigned group = pass_group(n, how_many);
   void* work = nullptr;
   if (needs_work(h->plan)) CFCHK(acquire_work(work_bytes(h->plan, n, group, d_sig, d_out), s, &work));
   struct WorkRelease {  // the workspace is marked busy on s whatever path returns
@@ -1556,35 +1566,55 @@ static int conv_device_impl(cf_spectrum_t h, const void* d_sig, void* d_out, uns
       if (w) release_work(s);
     }
   } wr{work, s};
+  // armed by cf_profile_begin: the last call of every group of prof_every (a
+  // call that follows others in the stream, not one that starts from an idle GPU)
+  const bool profiled = !times && g.prof_max > g.prof_calls && ++g.prof_seen % g.prof_every == 0;
   if (!times && !profiled)
     return run_conv(*f, h->plan, n, how_many, d_sig, d_out, work, h->d, hstride, scale, precision, s);
-  PassList p;
-  conv_passes(*f, h->plan, n, how_many, d_sig, d_out, work, h->d, hstride, scale, p, precision);
-  if (profiled) {
-    hipEvent_t* ev = &g.prof_ev[(size_t)g.prof_calls * (CF_MAX_PASSES + 1)];
-    CFCHK(run_passes(p, n, how_many, s, f->tw, ev));
-    if (g.prof_calls == 0) {
+  // the same groups, with events around every pass; a pass's time and bytes are
+  // summed over them
+  constexpr size_t kSet = CF_MAX_PASSES + 1;  // events of one group
+  const bool first = profiled && g.prof_calls == 0;
+  if (times) {
+    CFCHK(ensure_events());
+    memset(times, 0, sizeof *times);
+  }
+  const size_t V = cube_bytes(n);
+  for (unsigned b = 0; b < how_many; b += group) {
+    const unsigned nb = std::min(group, how_many - b);
+    PassList p;
+    conv_passes(*f, h->plan, n, nb, (const char*)d_sig + b * V, (char*)d_out + b * V, work,
+                (const char*)h->d + (size_t)b * hstride * 8, hstride, scale, p, precision);
+    hipEvent_t* ev = g.ev;
+    if (profiled) {
+      // one set per recorded call is there already; further groups of a call add theirs
+      while (g.prof_ev.size() < (g.prof_sets + 1) * kSet) {
+        hipEvent_t e = nullptr;
+        HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
+        g.prof_ev.push_back(e);
+      }
+      ev = &g.prof_ev[g.prof_sets++ * kSet];
+    }
+    CFCHK(run_passes(p, n, nb, s, f->tw, ev));
+    if (times) {
+      HIPCHK(hipEventSynchronize(ev[p.size()]));
+      times->npass = (unsigned)p.size();
+      for (size_t i = 0; i < p.size(); ++i) {
+        times->ms[i] += (float)ms_between(ev[i], ev[i + 1]);
+        snprintf(times->name[i], sizeof times->name[i], "%s", p[i].name);
+        times->bytes[i] += p[i].bytes;
+      }
+    } else if (first) {
       g.prof_npass = (unsigned)p.size();
-      g.prof_names.clear();
-      g.prof_bytes.clear();
-      for (auto& q : p) {
-        g.prof_names.push_back(q.name);
-        g.prof_bytes.push_back(q.bytes);
+      g.prof_names.resize(p.size());
+      g.prof_bytes.resize(p.size());
+      for (size_t i = 0; i < p.size(); ++i) {
+        g.prof_names[i] = p[i].name;
+        g.prof_bytes[i] = (b == 0 ? 0.0 : g.prof_bytes[i]) + p[i].bytes;
       }
     }
-    ++g.prof_calls;
-    return CF_OK;
   }
-  CFCHK(ensure_events());
-  CFCHK(run_passes(p, n, how_many, s, f->tw, g.ev));
-  HIPCHK(hipEventSynchronize(g.ev[p.size()]));
-  memset(times, 0, sizeof *times);
-  times->npass = (unsigned)p.size();
-  for (size_t i = 0; i < p.size(); ++i) {
-    times->ms[i] = (float)ms_between(g.ev[i], g.ev[i + 1]);
-    snprintf(times->name[i], sizeof times->name[i], "%s", p[i].name);
-    times->bytes[i] = p[i].bytes;
-  }
+  if (profiled) ++g.prof_calls;
   return CF_OK;
 }
 
@@ -1723,6 +1753,7 @@ extern "C" int cf_profile_begin(unsigned max_calls, unsigned every) {
   HIPCHK(hipStreamSynchronize(g.stream));
   g.prof_max = max_calls;
   g.prof_calls = 0;
+  g.prof_sets = 0;
   g.prof_every = every;
   g.prof_seen = 0;
   return CF_OK;
@@ -1736,12 +1767,12 @@ extern "C" int cf_profile_end(cf_pass_times_t* avg, unsigned* ncalls) {
   int rc = CF_OK;
   if (g.prof_calls > 0) {
     const size_t stride = CF_MAX_PASSES + 1;
-    hipEvent_t last = g.prof_ev[(size_t)(g.prof_calls - 1) * stride + g.prof_npass];
+    hipEvent_t last = g.prof_ev[(g.prof_sets - 1) * stride + g.prof_npass];
     if (hipEventSynchronize(last) != hipSuccess) rc = fail(CF_ERR_RUNTIME, "event synchronize failed");
     avg->npass = g.prof_npass;
     for (unsigned i = 0; i < g.prof_npass && rc == CF_OK; ++i) {
       double sum = 0.0;
-      for (unsigned c = 0; c < g.prof_calls; ++c)
+      for (size_t c = 0; c < g.prof_sets; ++c)
         sum += ms_between(g.prof_ev[c * stride + i], g.prof_ev[c * stride + i + 1]);
       avg->ms[i] = (float)(sum / g.prof_calls);
       snprintf(avg->name[i], sizeof avg->name[i], "%s", g.prof_names[i].c_str());
@@ -1751,6 +1782,7 @@ extern "C" int cf_profile_end(cf_pass_times_t* avg, unsigned* ncalls) {
   for (auto e : g.prof_ev) (void)hipEventDestroy(e);
   g.prof_ev.clear();
   g.prof_max = g.prof_calls = 0;
+  g.prof_sets = 0;
   return rc;
 }
 
@@ -1761,17 +1793,46 @@ extern "C" int cf_fft3d_device(unsigned n, const void* d_in, void* d_out, unsign
   CFCHK(require_ready());
   SizeFns* f = nullptr;
   CFCHK(size_res(n, &f));
+  hipStream_t s = (hipStream_t)stream;
   const unsigned group = pass_group(n, how_many);
+  // 256^3 in two passes through the workspace (97 us against 133 forward, 143
+  // inverse in one pass per axis).  A call recorded into a graph would share
+  // the workspace with whatever runs beside its replays, and cannot allocate
+  // it: it keeps the axis passes, as does a call that finds no memory for it.
+  void* work = nullptr;
+  if (n == 256) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusActive;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+      (void)hipGetLastError();
+      cap = hipStreamCaptureStatusActive;
+    }
+    if (cap == hipStreamCaptureStatusNone && acquire_work(g.fft_work, cube_bytes(n) * group, s, &work) != CF_OK) {
+      (void)hipGetLastError();
+      work = nullptr;
+    }
+  }
+  struct WorkRelease {
+    void* w;
+    hipStream_t s;
+    ~WorkRelease() {
+      if (w) release_work(g.fft_work, s);
+    }
+  } wr{work, s};
   for (unsigned b = 0; b < how_many; b += group) {
     const unsigned nb = std::min(group, how_many - b);
     const void* in = (const char*)d_in + b * cube_bytes(n);
     void* out = (char*)d_out + b * cube_bytes(n);
     PassList p;
-    if (inverse)
+    if (work) {
+      const double io = 2.0 * cube_bytes(n) * nb;
+      const int d = inverse ? 1 : 0;
+      p.push_back({f->fft2_first[d], cfgeo::fft2_first_tiles, cfgeo::fft2_first_threads, in, work, nullptr, 0, 1.0f, "yz1", io});
+      p.push_back({f->fft2_second[d], cfgeo::fft2_second_tiles, cfgeo::fft2_second_threads, work, out, nullptr, 0, 1.0f, "z2x", io});
+    } else if (inverse)
       inv_passes(*f, n, nb, in, out, 1.0f, p);
     else
       fwd_passes(*f, n, nb, in, out, p);
-    CFCHK(run_passes(p, n, nb, (hipStream_t)stream, f->tw, nullptr));
+    CFCHK(run_passes(p, n, nb, s, f->tw, nullptr));
   }
   return CF_OK;
 }

@@ -74,6 +74,10 @@ constexpr int split_c_tiles(int n, int v) { return n * ((n / 16) / split_gao(v))
 constexpr int split_b_threads(int n, int v) { return (n / 16) * split_gm(v) * (n / 16); }
 constexpr int split_b_tiles(int n, int v) { return 16 * (n / split_gm(v)); }
 
+// the plain 256^3 transform in two passes: tiles of (z2, 16 x), then of (k1, ky)
+constexpr int fft2_first_threads = 1024, fft2_first_tiles = 64 * 16;
+constexpr int fft2_second_threads = 1024, fft2_second_tiles = 4 * 256;
+
 // four-step variants the persistent batch kernel runs (outer tiles of 2 y2
 // values with one row per thread, middle tiles of 2 x): g24m2 and g24m2h
 constexpr int kBatchSplitCount = 2;

@@ -13,6 +13,7 @@
 #include "axis_passes.h"
 #include "batch_kernel.h"
 #include "fft_core.h"
+#include "fft_two_pass.h"
 #include "small_cube.h"
 #include "three_pass.h"
 #include "split_mfma.h"
@@ -227,6 +228,20 @@ struct SplitGeoCheckAll<N, cfgeo::kSplitVariants> {
   static constexpr bool ok = true;
 };
 static_assert(SplitGeoCheckAll<256>::ok && SplitGeoCheckAll<128>::ok, "split geometry");
+
+// ---- the plain 256^3 transform in two passes (fft_two_pass.h) -----------------------
+#define CF_FFT2(NAME, INV)                                                                                       \
+  extern "C" __global__ __launch_bounds__(cfgeo::fft2_first_threads) void cf_fft2_first_##NAME##_256(CF_ARGS) {  \
+    cfk::fft2_first_kernel<INV>(in, out, tw, ntotal);                                                            \
+  }                                                                                                              \
+  extern "C" __global__ __launch_bounds__(cfgeo::fft2_second_threads) void cf_fft2_second_##NAME##_256(CF_ARGS) { \
+    cfk::fft2_second_kernel<INV>(in, out, tw, ntotal);                                                           \
+  }
+CF_FFT2(fwd, false)
+CF_FFT2(inv, true)
+static_assert(cfk::Fft2Geo::A_THREADS == cfgeo::fft2_first_threads && cfk::Fft2Geo::A_TILES == cfgeo::fft2_first_tiles &&
+                  cfk::Fft2Geo::B_THREADS == cfgeo::fft2_second_threads && cfk::Fft2Geo::B_TILES == cfgeo::fft2_second_tiles,
+              "two-pass transform geometry");
 
 // ---- split-FP16 MFMA form of the four-step passes (split_mfma.h) ----------------------
 // outer passes GA = 2 over an intermediate of x group 4, middle tiles of 2 x:

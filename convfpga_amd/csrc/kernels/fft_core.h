@@ -263,6 +263,29 @@ __device__ __forceinline__ void xpose_quad_stage(float2 (&a)[16], bool set) {
       a[i + S] = set ? a[i + S] : y;
     }
 }
+// swap for lane bit 4 (B = 0) or 5 (B = 1) of registers i and i + S
+template <int B, int S>
+__device__ __forceinline__ void xpose_swap_stage(float2 (&a)[16]) {
+  // the lanes of lo with the bit set <-> those of hi with it clear
+  auto swap = [](float& lo, float& hi) {
+    const unsigned l = __builtin_bit_cast(unsigned, lo), h = __builtin_bit_cast(unsigned, hi);
+    if constexpr (B == 0) {
+      auto r = __builtin_amdgcn_permlane16_swap(l, h, false, false);
+      lo = __builtin_bit_cast(float, (unsigned)r[0]);
+      hi = __builtin_bit_cast(float, (unsigned)r[1]);
+    } else {
+      auto r = __builtin_amdgcn_permlane32_swap(l, h, false, false);
+      lo = __builtin_bit_cast(float, (unsigned)r[0]);
+      hi = __builtin_bit_cast(float, (unsigned)r[1]);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    if (!(i & S)) {
+      swap(a[i].x, a[i + S].x);
+      swap(a[i].y, a[i + S].y);
+    }
+}
 __device__ __forceinline__ void xpose16_rows(float2 (&a)[16], int t) {
   xpose_bank_stage<1, 8>(a);
   xpose_bank_stage<0, 4>(a);

@@ -46,3 +46,30 @@ def test_groups_equal_single_cubes(gpu, n, count, in_place):
         assert _same(one, tr[k]), k
         alone.close()
     batch.close()
+
+
+def test_timed_and_profiled_calls_run_the_groups(gpu):
+    """cf_conv3d_device_timed and cf_profile_* sum a pass over the groups of a
+    call: the bytes of 17 single cubes, the same output."""
+    import torch
+    api = gpu.api
+    n, count = 128, 17
+    print("case timed groups N=%d count=%d" % (n, count), flush=True)
+    sig = torch.empty((count, n ** 3), dtype=torch.complex64, device="cuda")
+    api.fill_uniform(sig, 2 * sig.numel(), 63001)
+    spec = gpu.Spectrum(n, sig, count)
+    alone = gpu.Spectrum(n, sig[0])
+    want, out = torch.empty_like(sig), torch.empty_like(sig)
+    gpu.conv3d_device(spec, sig, want, count)
+    one = gpu.conv3d_device_timed(alone, sig[0], out[0])
+    many = gpu.conv3d_device_timed(spec, sig, out, count)
+    assert _same(out, want)
+    assert [p["name"] for p in many] == [p["name"] for p in one]
+    assert all(m["bytes"] == count * o["bytes"] and m["ms"] > o["ms"] > 0 for m, o in zip(many, one))
+    out.zero_()
+    api.profile_begin(4, 2)
+    for _ in range(5):
+        gpu.conv3d_device(spec, sig, out, count)
+    passes, calls = api.profile_end()
+    assert calls == 2 and _same(out, want)
+    assert all(p["bytes"] == m["bytes"] and p["ms"] > 0 for p, m in zip(passes, many))
