@@ -25,6 +25,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -117,6 +118,38 @@ struct Workspace {
   hipEvent_t ev = nullptr;
 };
 
+// true if calls on s are being recorded into a graph (or that cannot be told)
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusActive;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+// Device memory of a spectrum, and who may still be reading it: `stream` (if
+// used), or anyone (`many`: several streams, a recorded call, a batch, a caller
+// that took its address).
+struct SpecMem {
+  void* d = nullptr;
+  size_t bytes = 0;
+  hipStream_t stream = nullptr;
+  bool used = false, many = false;
+  void use(hipStream_t s) {
+    // (hipStreamPerThread is another stream in every thread)
+    many = many || s == hipStreamPerThread || (used && stream != s) || capturing(s);
+    used = true;
+    stream = s;
+  }
+};
+// Freed spectra kept for the next one of the same size.  hipMalloc and hipFree
+// of a 256^3 spectrum, with the device synchronisation of the latter, cost as
+// much as the transform and the convolution together: a convolution with a new
+// filter took 594 us at 256^3 (3.5 ms the first time) and 81 us at 64^3, with
+// kept memory 273 (285) and 34.  Oldest out first; given back when an
+// allocation fails and by fpga_final().
+constexpr size_t kSpecPoolBytes = size_t(1) << 30;
+constexpr size_t kSpecPoolBlocks = 4;
+
 struct Engine {
   std::recursive_mutex mu;
   bool ready = false;
@@ -148,6 +181,7 @@ struct Engine {
   Workspace fft_work;  // of the two-pass plain transform; of its own, so that a transform
                        // meets neither the convolutions of other streams nor a graph
                        // that holds the address of theirs
+  std::vector<SpecMem> spec_pool;
   std::string arch;
   // error-norm scratch
   void* d_err = nullptr;
@@ -179,12 +213,38 @@ std::string lower(const std::string& s) {
   return r;
 }
 
+// Gives kept spectra back, oldest first, until `blocks` of `bytes` in all are
+// left (hipFree waits for whoever still reads them).
+bool spec_pool_shrink(size_t blocks, size_t bytes) {
+  size_t total = 0;
+  for (const SpecMem& m : g.spec_pool) total += m.bytes;
+  bool any = false;
+  while (!g.spec_pool.empty() && (g.spec_pool.size() > blocks || total > bytes)) {
+    total -= g.spec_pool.front().bytes;
+    (void)hipFree(g.spec_pool.front().d);
+    g.spec_pool.erase(g.spec_pool.begin());
+    any = true;
+  }
+  return any;
+}
+
+// hipMalloc that gives the kept spectra back before it fails.
+hipError_t dev_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory && spec_pool_shrink(0, 0)) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
 void pipe_release();
 
 void release_all() {
   if (g.ready || g.stream) (void)hipSetDevice(g.device);
   if (g.stream) (void)hipStreamSynchronize(g.stream);
   pipe_release();
+  spec_pool_shrink(0, 0);
   for (auto& kv : g.sizes)
     if (kv.second.tw) (void)hipFree(kv.second.tw);
   g.sizes.clear();
@@ -373,7 +433,7 @@ int size_res(unsigned n, SizeFns** out) {
   // twiddles W_N^j; for N = 256 and 512 followed by the DFT16 operand table
   // of the split-FP16 kernels (2 x 64 lanes x 4 x 16 bytes)
   const size_t tw_bytes = (size_t)n * 8, table_bytes = n == 256 || n == 512 ? 8192 : 0;
-  HIPCHK(hipMalloc(&s.tw, tw_bytes + table_bytes));
+  HIPCHK(dev_malloc(&s.tw, tw_bytes + table_bytes));
   void* tw = s.tw;
   int nn = (int)n;
   void* args[] = {&tw, &nn};
@@ -654,7 +714,7 @@ int ensure_device(void** p, size_t* have, size_t need) {
   if (*p) (void)hipFree(*p);
   *p = nullptr;
   *have = 0;
-  hipError_t e = hipMalloc(p, need);
+  hipError_t e = dev_malloc(p, need);
   if (e != hipSuccess) return fail(CF_ERR_NOMEM, "hipMalloc(%zu): %s", need, hipGetErrorString(e));
   *have = need;
   return CF_OK;
@@ -775,7 +835,7 @@ int acquire_work(Workspace& w, size_t bytes, hipStream_t s, void** out) {
     w.d = nullptr;
     w.bytes = 0;
     w.used = false;
-    hipError_t e = hipMalloc(&w.d, bytes);
+    hipError_t e = dev_malloc(&w.d, bytes);
     if (e != hipSuccess) return fail(CF_ERR_NOMEM, "hipMalloc(%zu) for the workspace: %s", bytes, hipGetErrorString(e));
     w.bytes = bytes;
   }
@@ -846,7 +906,7 @@ int autotune(unsigned n, SizeFns* f) {
     if (out) (void)hipFree(out);
     if (H) (void)hipFree(H);
   };
-  if (hipMalloc(&sig, V) != hipSuccess || hipMalloc(&out, V) != hipSuccess || hipMalloc(&H, V) != hipSuccess) {
+  if (dev_malloc(&sig, V) != hipSuccess || dev_malloc(&out, V) != hipSuccess || dev_malloc(&H, V) != hipSuccess) {
     cleanup();
     return fail(CF_ERR_NOMEM, "autotune scratch allocation failed");
   }
@@ -1010,7 +1070,7 @@ int pipe_ready(size_t slot_bytes) {
     }
     gp.slots = nullptr;
     gp.slots_bytes = 0;
-    const hipError_t e = hipMalloc(&gp.slots, need);
+    const hipError_t e = dev_malloc(&gp.slots, need);
     if (e != hipSuccess) return fail(CF_ERR_NOMEM, "hipMalloc(%zu) for the batch slots: %s", need, hipGetErrorString(e));
     gp.slots_bytes = need;
   }
@@ -1414,8 +1474,37 @@ struct cf_spectrum_s {
   unsigned n = 0, count = 0;
   int plan = CF_PLAN_AXIS5;
   void* d = nullptr;
-  bool view = false;  // aliases one filter of another handle's memory
+  bool view = false;             // aliases one filter of another handle's memory
+  std::shared_ptr<SpecMem> mem;  // that memory (a view's: its parent's)
 };
+
+// Memory for a spectrum that stream s will write: a kept block of the size, if
+// there is one and (unless only s can still be reading it) after waiting for
+// the device; otherwise new.
+static int spec_mem_get(size_t bytes, hipStream_t s, SpecMem* m) {
+  for (size_t i = 0; i < g.spec_pool.size(); ++i) {
+    if (g.spec_pool[i].bytes != bytes) continue;
+    const SpecMem old = g.spec_pool[i];
+    if (old.many || (old.used && (old.stream != s || s == hipStreamPerThread))) HIPCHK(hipDeviceSynchronize());
+    g.spec_pool.erase(g.spec_pool.begin() + i);
+    m->d = old.d;
+    m->bytes = bytes;
+    return CF_OK;
+  }
+  const hipError_t e = dev_malloc(&m->d, bytes);
+  if (e != hipSuccess) return fail(CF_ERR_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+  m->bytes = bytes;
+  return CF_OK;
+}
+
+static void spec_mem_put(const SpecMem& m) {
+  if (!g.ready || m.bytes > kSpecPoolBytes) {
+    (void)hipFree(m.d);
+    return;
+  }
+  g.spec_pool.push_back(m);
+  spec_pool_shrink(kSpecPoolBlocks, kSpecPoolBytes);
+}
 
 extern "C" const char* cf_last_error(void) { return g_err.c_str(); }
 
@@ -1434,11 +1523,14 @@ extern "C" int cf_spectrum_create(unsigned n, unsigned count, const void* filter
   h->n = n;
   h->count = count;
   const size_t bytes = cube_bytes(n) * count;
-  hipError_t e = hipMalloc(&h->d, bytes);
-  if (e != hipSuccess) {
+  h->mem = std::make_shared<SpecMem>();
+  const int got = spec_mem_get(bytes, s, h->mem.get());
+  if (got != CF_OK) {
     delete h;
-    return fail(CF_ERR_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+    return got;
   }
+  h->d = h->mem->d;
+  hipError_t e = hipSuccess;
   const void* src = filters;
   if (!on_device) {
     e = hipMemcpyAsync(h->d, filters, bytes, hipMemcpyHostToDevice, s);
@@ -1471,7 +1563,7 @@ extern "C" void cf_spectrum_destroy(cf_spectrum_t h) {
   if (!h) return;
   if (h->d && !h->view) {
     (void)hipSetDevice(g.device);
-    (void)hipFree(h->d);
+    spec_mem_put(*h->mem);
   }
   delete h;
 }
@@ -1486,11 +1578,17 @@ extern "C" int cf_spectrum_view(cf_spectrum_t parent, unsigned index, cf_spectru
   h->plan = parent->plan;
   h->d = (char*)parent->d + (size_t)index * cube_bytes(parent->n);
   h->view = true;
+  h->mem = parent->mem;
   *out = h;
   return CF_OK;
 }
 
-extern "C" const void* cf_spectrum_data(cf_spectrum_t h) { return h ? h->d : nullptr; }
+extern "C" const void* cf_spectrum_data(cf_spectrum_t h) {
+  std::lock_guard<std::recursive_mutex> lk(g.mu);
+  if (!h) return nullptr;
+  h->mem->many = true;  // the caller may read it on any stream
+  return h->d;
+}
 extern "C" int cf_spectrum_plan(cf_spectrum_t h) { return h ? h->plan : CF_ERR_ARG; }
 
 extern "C" int cf_plan_supported(unsigned n, int plan) { return plan_ok(n, plan) ? 1 : 0; }
@@ -1556,6 +1654,7 @@ static int conv_device_impl(cf_spectrum_t h, const void* d_sig, void* d_out, uns
   const float scale = scale_mode == CF_SCALE_INV_N3 ? (float)(1.0 / (double)cube_elems(n)) : 1.0f;
   const long long hstride = h->count == 1 ? 0 : (long long)cube_elems(n);
   hipStream_t s = (hipStream_t)stream;
+  h->mem->use(s);
   const unsigned group = pass_group(n, how_many);
   void* work = nullptr;
   if (needs_work(h->plan)) CFCHK(acquire_work(work_bytes(h->plan, n, group, d_sig, d_out), s, &work));
@@ -1652,6 +1751,7 @@ extern "C" int cf_conv3d_device_noalloc(cf_spectrum_t h, const void* d_sig, void
   }
   const float scale = scale_mode == CF_SCALE_INV_N3 ? (float)(1.0 / (double)cube_elems(n)) : 1.0f;
   const long long hstride = h->count == 1 ? 0 : (long long)cube_elems(n);
+  h->mem->use((hipStream_t)stream);
   return run_conv(f, h->plan, n, how_many, d_sig, d_out, work, h->d, hstride, scale, precision, (hipStream_t)stream);
 }
 
@@ -1695,6 +1795,7 @@ extern "C" int cf_conv3d_share_timed(cf_spectrum_t h, const void* d_sig, void* d
   CFCHK(size_res(h->n, &f));
   const unsigned n = h->n;
   hipStream_t s = (hipStream_t)stream;
+  h->mem->use(s);
   void* work = nullptr;
   if (needs_work(h->plan)) CFCHK(acquire_work(work_bytes(h->plan, n, 1, d_sig, d_out), s, &work));
   struct WorkRelease {
@@ -1801,12 +1902,7 @@ extern "C" int cf_fft3d_device(unsigned n, const void* d_in, void* d_out, unsign
   // it: it keeps the axis passes, as does a call that finds no memory for it.
   void* work = nullptr;
   if (n == 256) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusActive;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
-      (void)hipGetLastError();
-      cap = hipStreamCaptureStatusActive;
-    }
-    if (cap == hipStreamCaptureStatusNone && acquire_work(g.fft_work, cube_bytes(n) * group, s, &work) != CF_OK) {
+    if (!capturing(s) && acquire_work(g.fft_work, cube_bytes(n) * group, s, &work) != CF_OK) {
       (void)hipGetLastError();
       work = nullptr;
     }
@@ -1986,6 +2082,7 @@ static int batch_create(const cf_instance_t* inst, unsigned count, int scale_mod
     if (!x.d_sig || !x.d_out || !x.h) return fail(CF_ERR_ARG, "instance %u: NULL pointer", i);
     if (x.h->count != 1) return fail(CF_ERR_ARG, "instance %u: spectrum must hold one filter", i);
     CFCHK(size_res(x.h->n, &fns[i]));
+    x.h->mem->many = true;  // launches read it on any stream
     if (mode == CF_BATCH_PERSISTENT) {
       if (x.h->n < 16 || x.h->n > 256)
         return fail(CF_ERR_SIZE, "instance %u: the persistent batch runs edges 16..256, not %u", i, x.h->n);
@@ -2035,7 +2132,7 @@ static int batch_create(const cf_instance_t* inst, unsigned count, int scale_mod
       work_need += work_bytes(inst[i].h->plan, inst[i].h->n, 1, inst[i].d_sig, inst[i].d_out);
     }
     if (work_need) {
-      const hipError_t e = hipMalloc(&b->d_work, work_need);
+      const hipError_t e = dev_malloc(&b->d_work, work_need);
       if (e != hipSuccess) {
         batch_free(b);
         return fail(CF_ERR_NOMEM, "batch workspace: %s", hipGetErrorString(e));
@@ -2174,8 +2271,8 @@ static int batch_create(const cf_instance_t* inst, unsigned count, int scale_mod
     const int nitems = item;
     const size_t seg_bytes = sizeof(CfBatchSeg) * segs.size();
     const size_t tab_bytes = sizeof(int) * item_tab.size();
-    hipError_t e = hipMalloc(&b->d_segs, seg_bytes + sizeof stage_need + sizeof stage_first + tab_bytes);
-    if (e == hipSuccess) e = hipMalloc((void**)&b->d_ctr, sizeof(unsigned) * kBatchCounters * kBatchCtrStride);
+    hipError_t e = dev_malloc(&b->d_segs, seg_bytes + sizeof stage_need + sizeof stage_first + tab_bytes);
+    if (e == hipSuccess) e = dev_malloc((void**)&b->d_ctr, sizeof(unsigned) * kBatchCounters * kBatchCtrStride);
     if (e == hipSuccess) e = hipMemcpy(b->d_segs, segs.data(), seg_bytes, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy((char*)b->d_segs + seg_bytes, stage_need, sizeof stage_need, hipMemcpyHostToDevice);
     if (e == hipSuccess)
@@ -2235,7 +2332,7 @@ static int batch_create(const cf_instance_t* inst, unsigned count, int scale_mod
       i += run;
     }
     if (work_need) {
-      const hipError_t e = hipMalloc(&b->d_work, work_need);
+      const hipError_t e = dev_malloc(&b->d_work, work_need);
       if (e != hipSuccess) {
         batch_free(b);
         return fail(CF_ERR_NOMEM, "batch workspace: %s", hipGetErrorString(e));

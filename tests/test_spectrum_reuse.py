@@ -1,0 +1,55 @@
+"""Spectra made in memory that an earlier, destroyed spectrum of the same size
+used: the convolutions still queued with the old one, on the same or on another
+stream, keep its values, and the kept memory is bounded."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(x):
+    import torch
+    return torch.view_as_real(x).view(torch.int32)
+
+
+@pytest.mark.parametrize("n", [32, 128, 256])
+@pytest.mark.parametrize("other_stream", [False, True])
+def test_new_spectrum_waits_for_the_old_one(gpu, n, other_stream):
+    import torch
+    api = gpu.api
+    print("case spectrum reuse N=%d other_stream=%s" % (n, other_stream), flush=True)
+    P, rounds = n ** 3, 6
+    filt = torch.empty((rounds, P), dtype=torch.complex64, device="cuda")
+    sig = torch.empty(P, dtype=torch.complex64, device="cuda")
+    api.fill_uniform(filt, 2 * filt.numel(), 64001 + n)
+    api.fill_uniform(sig, 2 * P, 64002 + n)
+    keep = [gpu.Spectrum(n, filt[k]) for k in range(rounds)]
+    want = torch.empty_like(filt)
+    for k in range(rounds):
+        gpu.conv3d_device(keep[k], sig, want[k])
+    torch.cuda.synchronize()
+    for s in keep:
+        s.close()
+    out = torch.empty_like(filt)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for k in range(rounds):  # each closed with its convolution still queued
+        st = streams[k % 2 if other_stream else 0]
+        spec = gpu.Spectrum(n, filt[k], stream=st)
+        gpu.conv3d_device(spec, sig, out[k], stream=st)
+        spec.close()
+    torch.cuda.synchronize()
+    assert torch.equal(_bits(out), _bits(want))
+
+
+def test_kept_memory_is_bounded(gpu):
+    import torch
+    n, count = 256, 2
+    print("case spectrum memory bound", flush=True)
+    filt = torch.zeros((count, n ** 3), dtype=torch.complex64, device="cuda")
+    torch.cuda.synchronize()
+    gpu.Spectrum(n, filt, count).close()  # (workspace and tables are there)
+    free0 = torch.cuda.mem_get_info()[0]
+    specs = [gpu.Spectrum(n, filt, count) for _ in range(8)]  # 2 GiB
+    for s in specs:
+        s.close()
+    assert free0 - torch.cuda.mem_get_info()[0] <= 1 << 30
