@@ -68,6 +68,7 @@ struct SizeFns {
   hipFunction_t colz_fwd = nullptr, colz_inv = nullptr, colz_conv = nullptr;
   hipFunction_t cube_fwd = nullptr, cube_inv = nullptr, cube_conv = nullptr;  // N in {8, 16}: a cube per work-group
   hipFunction_t plane_fwd = nullptr, plane_inv = nullptr;                 // N in {32, 64, 128}
+  hipFunction_t rows_fwd = nullptr, rows_inv = nullptr, mid_split = nullptr;  // N = 64, one cube of the plane plan
   hipFunction_t coly_fwd_zb = nullptr, coly_inv_zb = nullptr, colz_fwd_zb = nullptr, colz_conv_zb = nullptr;  // N >= 64
   hipFunction_t xy1_fwd[cfgeo::kSplitVariants] = {}, xy1_inv[cfgeo::kSplitVariants] = {};  // N = 256
   hipFunction_t mid[cfgeo::kSplitVariants] = {}, mspec[cfgeo::kSplitVariants] = {};
@@ -410,6 +411,11 @@ int size_res(unsigned n, SizeFns** out) {
     snprintf(name, sizeof name, "cf_midspec_%u_%s", n, sfx);
     CFCHK(get_fn(&s.mspec[vi], name));
   }
+  if (n == 64) {
+    CFCHK(get_fn(&s.rows_fwd, "cf_rows_fwd_64"));
+    CFCHK(get_fn(&s.rows_inv, "cf_rows_inv_64"));
+    CFCHK(get_fn(&s.mid_split, "cf_mid_64"));
+  }
   if (n == 256) {
     CFCHK(get_fn(&s.fft2_first[0], "cf_fft2_first_fwd_256"));
     CFCHK(get_fn(&s.fft2_first[1], "cf_fft2_first_inv_256"));
@@ -543,12 +549,14 @@ void inv_passes(const SizeFns& f, unsigned n, unsigned nb, const void* in, void*
 // Convolution passes of `plan`.  AXIS5: x, y, z*H*z, y^-1, x^-1(+scale), in
 // place in out.  PLANE3: xy-plane, z*H*z, xy-plane^-1(+scale), in place.
 // SPLIT3: sig -> work (pass A), work in place (middle), work -> out (pass C).
-// AXIS5 at N = 8 and 16: one pass over whole cubes, unless the caller reports
-// the forward and the inverse half separately (same bits either way).
+// Small cubes have other forms of the same transforms (same bits): AXIS5 at N = 8
+// and 16 one pass over whole cubes, PLANE3 for one 64^3 cube smaller tiles with y
+// split over the passes.  own_passes: the plan's own passes in any case, for
+// callers that report its forward and inverse half, or its tiles, by themselves.
 // Returns the index of the first pass after the product (the fpga_t split).
 size_t conv_passes(const SizeFns& f, int plan, unsigned n, unsigned nb, const void* sig, void* out, void* work,
                    const void* H, long long hstride, float scale, PassList& v,
-                   int precision = CF_PREC_FP32, bool separate_inverse = false) {
+                   int precision = CF_PREC_FP32, bool own_passes = false) {
   const double V = (double)cube_bytes(n);
   const double io = 2.0 * V * nb;
   const double hbytes = hstride ? V * nb : V;
@@ -580,6 +588,15 @@ size_t conv_passes(const SizeFns& f, int plan, unsigned n, unsigned nb, const vo
   }
   const unsigned rt = cfgeo::row_threads(n), rT = cfgeo::row_tiles(n);
   const unsigned ct = cfgeo::col_threads(n), cT = cfgeo::col_tiles(n);
+  if (plan == CF_PLAN_PLANE3 && n == 64 && nb == 1 && !own_passes) {
+    const unsigned rt64 = cfgeo::rows64_threads, rT64 = cfgeo::rows64_groups;
+    v.push_back({f.rows_fwd, rT64, rt64, sig, out, nullptr, 0, 1.0f, "xy1_fwd", io});
+    v.push_back({f.mid_split, cfgeo::mid64_tiles, cfgeo::mid64_threads, out, out, H, hstride, 1.0f, "y2z_fwd_mul_inv",
+                 io + hbytes});
+    const size_t split = v.size();
+    v.push_back({f.rows_inv, rT64, rt64, out, out, nullptr, 0, scale, "xy1_inv", io});
+    return split;
+  }
   if (plan == CF_PLAN_PLANE3) {
     const unsigned pt = cfgeo::plane_threads(n), pT = cfgeo::plane_tiles(n);
     v.push_back({f.plane_fwd, pT, pt, sig, out, nullptr, 0, 1.0f, "xy_fwd", io});
@@ -617,7 +634,7 @@ size_t conv_passes(const SizeFns& f, int plan, unsigned n, unsigned nb, const vo
     v.push_back({f.row_inv, rT, rt, out, out, nullptr, 0, scale, "x_inv", io});
     return split;
   }
-  if (cfgeo::cube_supported((int)n) && !separate_inverse) {
+  if (cfgeo::cube_supported((int)n) && !own_passes) {
     v.push_back({f.cube_conv, 1, n * n, sig, out, H, hstride, scale, "xyz_fwd_mul_inv", io + hbytes});
     return v.size();
   }
@@ -1806,7 +1823,7 @@ extern "C" int cf_conv3d_share_timed(cf_spectrum_t h, const void* d_sig, void* d
     }
   } wr{work, s};
   PassList p;
-  conv_passes(*f, h->plan, n, 1, d_sig, d_out, work, h->d, 0, (float)(1.0 / (double)cube_elems(n)), p, precision);
+  conv_passes(*f, h->plan, n, 1, d_sig, d_out, work, h->d, 0, (float)(1.0 / (double)cube_elems(n)), p, precision, true);
   // every work-group count stays a multiple of 8 x the widest sibling group (8)
   for (const Pass& q : p)
     if (shares > 1 && q.tiles % (shares * 64) != 0)

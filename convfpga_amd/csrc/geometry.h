@@ -74,6 +74,11 @@ constexpr int split_c_tiles(int n, int v) { return n * ((n / 16) / split_gao(v))
 constexpr int split_b_threads(int n, int v) { return (n / 16) * split_gm(v) * (n / 16); }
 constexpr int split_b_tiles(int n, int v) { return 16 * (n / split_gm(v)); }
 
+// one 64^3 cube of the plane plan with y split over the passes: row passes of four
+// one-wave tiles per work-group, middle tiles of 2 x
+constexpr int rows64_threads = 256, rows64_groups = 128;
+constexpr int mid64_threads = 128, mid64_tiles = 256;
+
 // the plain 256^3 transform in two passes: tiles of (z2, 16 x), then of (k1, ky)
 constexpr int fft2_first_threads = 1024, fft2_first_tiles = 64 * 16;
 constexpr int fft2_second_threads = 1024, fft2_second_tiles = 4 * 256;

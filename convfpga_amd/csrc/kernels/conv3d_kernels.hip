@@ -14,6 +14,7 @@
 #include "batch_kernel.h"
 #include "fft_core.h"
 #include "fft_two_pass.h"
+#include "plane_split.h"
 #include "small_cube.h"
 #include "three_pass.h"
 #include "split_mfma.h"
@@ -228,6 +229,21 @@ struct SplitGeoCheckAll<N, cfgeo::kSplitVariants> {
   static constexpr bool ok = true;
 };
 static_assert(SplitGeoCheckAll<256>::ok && SplitGeoCheckAll<128>::ok, "split geometry");
+
+// ---- one 64^3 cube of the plane plan, y split over the passes (plane_split.h) ------------
+extern "C" __global__ __launch_bounds__(cfgeo::rows64_threads) void cf_rows_fwd_64(CF_ARGS) {
+  cfk::rows64_kernel<false>(in, out, tw, scale, ntotal);
+}
+extern "C" __global__ __launch_bounds__(cfgeo::rows64_threads) void cf_rows_inv_64(CF_ARGS) {
+  cfk::rows64_kernel<true>(in, out, tw, scale, ntotal);
+}
+extern "C" __global__ __launch_bounds__(cfgeo::mid64_threads) void cf_mid_64(CF_ARGS) {
+  cfk::mid64_kernel(in, out, H, tw, hstride, ntotal);
+}
+static_assert(cfk::PlaneSplit::THREADS == cfgeo::rows64_threads &&
+                  cfk::PlaneSplit::TILES == cfgeo::rows64_groups * cfk::PlaneSplit::WAVES &&
+                  cfk::MidSplit::THREADS == cfgeo::mid64_threads && cfk::MidSplit::TILES == cfgeo::mid64_tiles,
+              "split plane geometry");
 
 // ---- the plain 256^3 transform in two passes (fft_two_pass.h) -----------------------
 #define CF_FFT2(NAME, INV)                                                                                       \
