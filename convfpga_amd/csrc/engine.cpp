@@ -2337,7 +2337,12 @@ static int batch_create(const cf_instance_t* inst, unsigned count, int scale_mod
       const size_t V = cube_bytes(n);
       unsigned run = 1;
       const bool shared = i + 1 < count && inst[i + 1].h == inst[i].h;
-      while (i + run < count && inst[i + run].h->n == n && inst[i + run].h->plan == inst[i].h->plan &&
+      // the cubes of one pass sequence run at the same time, so none may write
+      // what another reads: an output that starts k cubes away from its signal
+      // (a chain of instances along one buffer) ends the run after k of them
+      const size_t apart = (size_t)std::abs((const char*)inst[i].d_out - (const char*)inst[i].d_sig) / V;
+      const size_t most = inst[i].d_out == inst[i].d_sig ? count : std::max<size_t>(1, apart);
+      while (run < most && i + run < count && inst[i + run].h->n == n && inst[i + run].h->plan == inst[i].h->plan &&
              (shared ? inst[i + run].h == inst[i].h
                      : (const char*)inst[i + run].h->d == (const char*)inst[i].h->d + run * V) &&
              (const char*)inst[i + run].d_sig == (const char*)inst[i].d_sig + run * V &&

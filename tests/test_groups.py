@@ -73,3 +73,29 @@ def test_timed_and_profiled_calls_run_the_groups(gpu):
     passes, calls = api.profile_end()
     assert calls == 2 and _same(out, want)
     assert all(p["bytes"] == m["bytes"] and p["ms"] > 0 for p, m in zip(passes, many))
+
+
+@pytest.mark.parametrize("n", [16, 64, 128])
+@pytest.mark.parametrize("step", [1, 2, -1])
+def test_graph_keeps_order_along_one_buffer(gpu, n, step):
+    """Graph instances whose signals and outputs follow each other in one buffer,
+    the output `step` cubes behind the signal: each reads what an earlier one
+    wrote (or writes what an earlier one has read), in the given order."""
+    import torch
+    api = gpu.api
+    print("case graph chain N=%d step=%d" % (n, step), flush=True)
+    P, count = n ** 3, 5
+    lead = max(0, -step)
+    buf = torch.empty((count + abs(step), P), dtype=torch.complex64, device="cuda")
+    api.fill_uniform(buf, 2 * buf.numel(), 65001 + n)
+    filt = torch.empty(P, dtype=torch.complex64, device="cuda")
+    api.fill_uniform(filt, 2 * P, 65002 + n)
+    spec = gpu.Spectrum(n, filt)
+    want = buf.clone()
+    for k in range(count):
+        gpu.conv3d_device(spec, want[lead + k], want[lead + k + step])
+    batch = api.Batch([(buf[lead + k], buf[lead + k + step], spec) for k in range(count)], mode=api.CF_BATCH_GRAPH)
+    batch.launch()
+    batch.check()
+    batch.close()
+    assert _same(buf, want)
