@@ -79,6 +79,18 @@ constexpr int split_b_tiles(int n, int v) { return 16 * (n / split_gm(v)); }
 constexpr int rows64_threads = 256, rows64_groups = 128;
 constexpr int mid64_threads = 128, mid64_tiles = 256;
 
+// a batch of 64^3 and one of 32^3 in one launch per pass of the plane plan
+constexpr int pair_threads = 512, pair_z_threads = 256;
+struct PairPart {
+  const void* in;
+  void* out;
+  const void* H;
+  const void* tw;
+  long long hstride;
+  float scale;
+  int groups;
+};
+
 // the plain 256^3 transform in two passes: tiles of (z2, 16 x), then of (k1, ky)
 constexpr int fft2_first_threads = 1024, fft2_first_tiles = 64 * 16;
 constexpr int fft2_second_threads = 1024, fft2_second_tiles = 4 * 256;

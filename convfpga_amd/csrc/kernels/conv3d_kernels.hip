@@ -14,6 +14,7 @@
 #include "batch_kernel.h"
 #include "fft_core.h"
 #include "fft_two_pass.h"
+#include "plane_pair.h"
 #include "plane_split.h"
 #include "small_cube.h"
 #include "three_pass.h"
@@ -244,6 +245,17 @@ static_assert(cfk::PlaneSplit::THREADS == cfgeo::rows64_threads &&
                   cfk::PlaneSplit::TILES == cfgeo::rows64_groups * cfk::PlaneSplit::WAVES &&
                   cfk::MidSplit::THREADS == cfgeo::mid64_threads && cfk::MidSplit::TILES == cfgeo::mid64_tiles,
               "split plane geometry");
+
+// ---- a 64^3 and a 32^3 batch of the plane plan in one launch per pass (plane_pair.h) -----
+extern "C" __global__ __launch_bounds__(cfgeo::pair_threads) void cf_pair_plane_fwd(cfk::PairPart a, cfk::PairPart b) {
+  cfk::pair_plane_kernel<false>(a, b);
+}
+extern "C" __global__ __launch_bounds__(cfgeo::pair_threads) void cf_pair_plane_inv(cfk::PairPart a, cfk::PairPart b) {
+  cfk::pair_plane_kernel<true>(a, b);
+}
+extern "C" __global__ __launch_bounds__(cfgeo::pair_z_threads) void cf_pair_colz_conv(cfk::PairPart a, cfk::PairPart b) {
+  cfk::pair_z_kernel(a, b);
+}
 
 // ---- the plain 256^3 transform in two passes (fft_two_pass.h) -----------------------
 #define CF_FFT2(NAME, INV)                                                                                       \

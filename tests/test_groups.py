@@ -99,3 +99,73 @@ def test_graph_keeps_order_along_one_buffer(gpu, n, step):
     batch.check()
     batch.close()
     assert _same(buf, want)
+
+
+@pytest.mark.parametrize("n32,n64", [(1, 1), (16, 8), (5, 3), (1, 9), (40, 1), (513, 2), (3, 65)])
+@pytest.mark.parametrize("first", [32, 64])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_graph_pairs_32_and_64(gpu, n32, n64, first, in_place):
+    """A 32^3 and a 64^3 run next to each other share their launches (run_pair,
+    engine.cpp), up to a group of each (512 and 64 cubes; one more and they run by
+    themselves): the bits of calls on the cubes alone, one filter each or shared."""
+    import torch
+    api = gpu.api
+    print("case pair 32:%d 64:%d first=%d in_place=%s" % (n32, n64, first, in_place), flush=True)
+    inst, want = [], []
+    for n, count in ((32, n32), (64, n64))[:: 1 if first == 32 else -1]:
+        sig = torch.empty((count, n ** 3), dtype=torch.complex64, device="cuda")
+        filt = torch.empty_like(sig)
+        api.fill_uniform(sig, 2 * sig.numel(), 64000 + n + count)
+        api.fill_uniform(filt, 2 * filt.numel(), 65000 + n + count)
+        spec = gpu.Spectrum(n, filt, count if n == 32 else 1)
+        ref = torch.empty_like(sig)
+        gpu.conv3d_device(spec, sig, ref, count)
+        out = sig if in_place else torch.zeros_like(sig)
+        inst += [(sig[k], out[k], spec.view(k) if n == 32 else spec) for k in range(count)]
+        want.append((out, ref))
+    batch = api.Batch(inst, mode=api.CF_BATCH_GRAPH)
+    batch.launch()
+    batch.check()
+    for out, ref in want:
+        assert _same(out, ref)
+    if not in_place:
+        for _ in range(2):
+            for out, _ref in want:
+                out.zero_()
+            batch.launch()
+            for out, ref in want:
+                assert _same(out, ref)
+    batch.close()
+
+
+@pytest.mark.parametrize("overlap", ["out_sig", "out_out", "sig_out"])
+def test_graph_pair_keeps_order(gpu, overlap):
+    """A 64^3 and a 32^3 instance that meet in memory run one after the other."""
+    import torch
+    api = gpu.api
+    print("case pair order %s" % overlap, flush=True)
+    a, c = 64 ** 3, 32 ** 3
+    buf = torch.empty(4 * a, dtype=torch.complex64, device="cuda")
+    big, small = torch.empty(a, dtype=torch.complex64, device="cuda"), torch.empty(c, dtype=torch.complex64, device="cuda")
+    for k, t in enumerate((buf, big, small)):
+        api.fill_uniform(t, 2 * t.numel(), 66000 + k)
+    hb, hs = gpu.Spectrum(64, big), gpu.Spectrum(32, small)
+
+    def at(b, off, n):
+        return b[off:off + n]
+
+    def insts(b):
+        lo, mid, tail = a - c, a + c, 2 * a
+        if overlap == "out_sig":      # the second reads the end of the first's output
+            return [(at(b, tail, a), at(b, 0, a), hb), (at(b, lo, c), at(b, 3 * a, c), hs)]
+        if overlap == "out_out":      # both write the end of the first's output
+            return [(at(b, tail, a), at(b, 0, a), hb), (at(b, 3 * a, c), at(b, lo, c), hs)]
+        return [(at(b, mid, a), at(b, tail, a), hb), (at(b, 3 * a, c), at(b, mid, c), hs)]  # writes what the first read
+    ref = buf.clone()
+    for s, o, h in insts(ref):
+        gpu.conv3d_device(h, s, o)
+    batch = api.Batch(insts(buf), mode=api.CF_BATCH_GRAPH)
+    batch.launch()
+    batch.check()
+    assert _same(buf, ref)
+    batch.close()
