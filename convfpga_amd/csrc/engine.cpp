@@ -69,6 +69,7 @@ struct SizeFns {
   hipFunction_t cube_fwd = nullptr, cube_inv = nullptr, cube_conv = nullptr;  // N in {8, 16}: a cube per work-group
   hipFunction_t plane_fwd = nullptr, plane_inv = nullptr;                 // N in {32, 64, 128}
   hipFunction_t rows_fwd = nullptr, rows_inv = nullptr, mid_split = nullptr;  // N = 64, one cube of the plane plan
+  hipFunction_t coly_fwd_slab = nullptr, colz_conv_slab = nullptr, coly_inv_slab = nullptr;  // N = 512, by x slabs
   hipFunction_t coly_fwd_zb = nullptr, coly_inv_zb = nullptr, colz_fwd_zb = nullptr, colz_conv_zb = nullptr;  // N >= 64
   hipFunction_t xy1_fwd[cfgeo::kSplitVariants] = {}, xy1_inv[cfgeo::kSplitVariants] = {};  // N = 256
   hipFunction_t mid[cfgeo::kSplitVariants] = {}, mspec[cfgeo::kSplitVariants] = {};
@@ -151,6 +152,8 @@ struct SpecMem {
 constexpr size_t kSpecPoolBytes = size_t(1) << 30;
 constexpr size_t kSpecPoolBlocks = 4;
 
+constexpr size_t kMaxLaunches = 16;  // of one convolution of a group of cubes (PassList)
+
 struct Engine {
   std::recursive_mutex mu;
   bool ready = false;
@@ -188,23 +191,24 @@ struct Engine {
   // error-norm scratch
   void* d_err = nullptr;
   size_t d_err_bytes = 0;
-  hipEvent_t ev[CF_MAX_PASSES + 8] = {};
+  hipEvent_t ev[kMaxLaunches + 8] = {};
   // device address of the code object's cf_scratch array on g.device (the
   // only device this engine drives), looked up once when the module is loaded
   void* scratch = nullptr;
   size_t scratch_bytes = 0;
-  // cf_profile_begin/end: sets of CF_MAX_PASSES+1 events, at least one for each of up to prof_max calls
+  // cf_profile_begin/end: sets of kMaxLaunches+1 events, at least one for each of up to prof_max calls
   std::vector<hipEvent_t> prof_ev;
   unsigned prof_max = 0, prof_calls = 0, prof_npass = 0;
   size_t prof_sets = 0;  // sets of events recorded: one per group of cubes of each recorded call
   unsigned prof_every = 1, prof_seen = 0;  // record the last call of every group of prof_every while armed
   std::vector<std::string> prof_names;
+  std::vector<unsigned> prof_slot;  // pass of each launch of a set
   std::vector<double> prof_bytes;
 };
 
 Engine g;
 constexpr int kErrBlocks = 1024;
-constexpr int kNumEvents = CF_MAX_PASSES + 8;
+constexpr int kNumEvents = kMaxLaunches + 8;
 
 size_t cube_elems(unsigned n) { return (size_t)n * n * n; }
 size_t cube_bytes(unsigned n) { return cube_elems(n) * 8; }
@@ -432,6 +436,9 @@ int size_res(unsigned n, SizeFns** out) {
     CFCHK(get_fn(&s.mx_coly_fwd, "cf_coly_fwd_512_s"));
     CFCHK(get_fn(&s.mx_coly_inv, "cf_coly_inv_512_s"));
     CFCHK(get_fn(&s.mx_colz_conv, "cf_colz_conv_512_s"));
+    CFCHK(get_fn(&s.coly_fwd_slab, "cf_coly_fwd_slab_512"));
+    CFCHK(get_fn(&s.colz_conv_slab, "cf_colz_conv_slab_512"));
+    CFCHK(get_fn(&s.coly_inv_slab, "cf_coly_inv_slab_512"));
     CFCHK(get_fn(&s.mx_coly_fwd_zb, "cf_coly_fwd_zb_512_s"));
     CFCHK(get_fn(&s.mx_colz_conv_zb, "cf_colz_conv_zb_512_s"));
     CFCHK(get_fn(&s.mx_coly_inv_zb, "cf_coly_inv_zb_512_s"));
@@ -466,17 +473,23 @@ struct Pass {
   float scale;
   const char* name;
   double bytes;  // algorithmic HBM bytes for the whole launch
+  unsigned slot = 0;  // the pass of the call it is (part of), for reports
 };
 
-// The passes of one call: at most CF_MAX_PASSES, held in place (building a
-// schedule touches no heap, so the allocation-free entry point allocates
-// nothing at all).
+// The launches of one call: at most kMaxLaunches, of at most CF_MAX_PASSES passes,
+// held in place (building a schedule touches no heap, so the allocation-free
+// entry point allocates nothing at all).
 struct PassList {
-  Pass p[CF_MAX_PASSES];
+  Pass p[kMaxLaunches];
   size_t n = 0;
-  void push_back(const Pass& x) {
-    if (n < CF_MAX_PASSES) p[n++] = x;  // every schedule here has at most 5 passes
+  void push_back(const Pass& x) { push_part(x, n ? p[n - 1].slot + 1 : 0); }
+  // a launch that does part of pass `slot`
+  void push_part(const Pass& x, unsigned slot) {
+    if (n >= kMaxLaunches) return;  // every schedule here has fewer
+    p[n] = x;
+    p[n++].slot = slot;
   }
+  unsigned slots() const { return n ? p[n - 1].slot + 1 : 0; }  // the last launch is of the last pass
   size_t size() const { return n; }
   Pass& operator[](size_t i) { return p[i]; }
   const Pass& operator[](size_t i) const { return p[i]; }
@@ -552,7 +565,8 @@ void inv_passes(const SizeFns& f, unsigned n, unsigned nb, const void* in, void*
 // SPLIT3: sig -> work (pass A), work in place (middle), work -> out (pass C).
 // Small cubes have other forms of the same transforms (same bits): AXIS5 at N = 8
 // and 16 one pass over whole cubes, PLANE3 for one 64^3 cube smaller tiles with y
-// split over the passes.  own_passes: the plan's own passes in any case, for
+// split over the passes, AXIS5Z for one 512^3 cube the y and z passes by slabs of
+// x.  own_passes: the plan's own passes in any case, for
 // callers that report its forward and inverse half, or its tiles, by themselves.
 // Returns the index of the first pass after the product (the fpga_t split).
 size_t conv_passes(const SizeFns& f, int plan, unsigned n, unsigned nb, const void* sig, void* out, void* work,
@@ -625,6 +639,22 @@ size_t conv_passes(const SizeFns& f, int plan, unsigned n, unsigned nb, const vo
     const size_t split = v.size();
     v.push_back({f.xy1_inv[vi], cT3, ct3, w2, out, nullptr, 0, scale, "xy1_inv", io});
     return split;
+  }
+  if (plan == CF_PLAN_AXIS5Z && n == 512 && nb == 1 && !own_passes) {
+    // the passes through the workspace one x slab after the other
+    v.push_back({f.row_fwd, rT, rt, sig, out, nullptr, 0, 1.0f, "x_fwd", io});
+    const unsigned sT = cfgeo::slab_tiles;
+    const double sio = io / cfgeo::slabs_512, sh = hbytes / cfgeo::slabs_512;
+    for (unsigned k = 0; k < (unsigned)cfgeo::slabs_512; ++k) {
+      const size_t x = (size_t)k * cfgeo::slab_groups * cfgeo::col_c(512);  // the slab's first column
+      char* o = (char*)out + x * 8;
+      const char* h = (const char*)H + x * 512 * 512 * 8;
+      v.push_part({f.coly_fwd_slab, sT, ct, o, work, nullptr, 0, 1.0f, "y_fwd", sio}, 1);
+      v.push_part({f.colz_conv_slab, sT, ct, work, work, h, hstride, 1.0f, "z_fwd_mul_z_inv", sio + sh}, 2);
+      v.push_part({f.coly_inv_slab, sT, ct, work, o, nullptr, 0, 1.0f, "y_inv", sio}, 3);
+    }
+    v.push_back({f.row_inv, rT, rt, out, out, nullptr, 0, scale, "x_inv", io});
+    return v.size() - 1;
   }
   if (plan == CF_PLAN_AXIS5Z) {  // natural -> z-blocked in the workspace -> natural
     v.push_back({f.row_fwd, rT, rt, sig, out, nullptr, 0, 1.0f, "x_fwd", io});
@@ -1722,7 +1752,7 @@ static int conv_device_impl(cf_spectrum_t h, const void* d_sig, void* d_out, uns
     return run_conv(*f, h->plan, n, how_many, d_sig, d_out, work, h->d, hstride, scale, precision, s);
   // the same groups, with events around every pass; a pass's time and bytes are
   // summed over them
-  constexpr size_t kSet = CF_MAX_PASSES + 1;  // events of one group
+  constexpr size_t kSet = kMaxLaunches + 1;  // events of one group
   const bool first = profiled && g.prof_calls == 0;
   if (times) {
     CFCHK(ensure_events());
@@ -1747,19 +1777,24 @@ static int conv_device_impl(cf_spectrum_t h, const void* d_sig, void* d_out, uns
     CFCHK(run_passes(p, n, nb, s, f->tw, ev));
     if (times) {
       HIPCHK(hipEventSynchronize(ev[p.size()]));
-      times->npass = (unsigned)p.size();
+      times->npass = p.slots();
       for (size_t i = 0; i < p.size(); ++i) {
-        times->ms[i] += (float)ms_between(ev[i], ev[i + 1]);
-        snprintf(times->name[i], sizeof times->name[i], "%s", p[i].name);
-        times->bytes[i] += p[i].bytes;
+        const unsigned k = p[i].slot;
+        times->ms[k] += (float)ms_between(ev[i], ev[i + 1]);
+        snprintf(times->name[k], sizeof times->name[k], "%s", p[i].name);
+        times->bytes[k] += p[i].bytes;
       }
     } else if (first) {
-      g.prof_npass = (unsigned)p.size();
-      g.prof_names.resize(p.size());
-      g.prof_bytes.resize(p.size());
-      for (size_t i = 0; i < p.size(); ++i) {
-        g.prof_names[i] = p[i].name;
-        g.prof_bytes[i] = (b == 0 ? 0.0 : g.prof_bytes[i]) + p[i].bytes;
+      if (b == 0) {
+        g.prof_npass = p.slots();
+        g.prof_names.assign(p.slots(), "");
+        g.prof_bytes.assign(p.slots(), 0.0);
+        g.prof_slot.clear();
+        for (const Pass& x : p) g.prof_slot.push_back(x.slot);
+      }
+      for (const Pass& x : p) {
+        g.prof_names[x.slot] = x.name;
+        g.prof_bytes[x.slot] += x.bytes;
       }
     }
   }
@@ -1893,7 +1928,7 @@ extern "C" int cf_profile_begin(unsigned max_calls, unsigned every) {
   if (every == 0 || every > 1000) return fail(CF_ERR_ARG, "every must be in 1..1000");
   CFCHK(require_ready());
   for (auto e : g.prof_ev) (void)hipEventDestroy(e);
-  g.prof_ev.assign((size_t)max_calls * (CF_MAX_PASSES + 1), nullptr);
+  g.prof_ev.assign((size_t)max_calls * (kMaxLaunches + 1), nullptr);
   // timing-only events: no system-scope fence (cache writeback) when they
   // complete, which would otherwise stall the next pass for microseconds
   for (auto& e : g.prof_ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
@@ -1917,14 +1952,15 @@ extern "C" int cf_profile_end(cf_pass_times_t* avg, unsigned* ncalls) {
   *ncalls = g.prof_calls;
   int rc = CF_OK;
   if (g.prof_calls > 0) {
-    const size_t stride = CF_MAX_PASSES + 1;
-    hipEvent_t last = g.prof_ev[(g.prof_sets - 1) * stride + g.prof_npass];
+    const size_t stride = kMaxLaunches + 1, launches = g.prof_slot.size();
+    hipEvent_t last = g.prof_ev[(g.prof_sets - 1) * stride + launches];
     if (hipEventSynchronize(last) != hipSuccess) rc = fail(CF_ERR_RUNTIME, "event synchronize failed");
     avg->npass = g.prof_npass;
     for (unsigned i = 0; i < g.prof_npass && rc == CF_OK; ++i) {
       double sum = 0.0;
       for (size_t c = 0; c < g.prof_sets; ++c)
-        sum += ms_between(g.prof_ev[c * stride + i], g.prof_ev[c * stride + i + 1]);
+        for (size_t k = 0; k < launches; ++k)
+          if (g.prof_slot[k] == i) sum += ms_between(g.prof_ev[c * stride + k], g.prof_ev[c * stride + k + 1]);
       avg->ms[i] = (float)(sum / g.prof_calls);
       snprintf(avg->name[i], sizeof avg->name[i], "%s", g.prof_names[i].c_str());
       avg->bytes[i] = g.prof_bytes[i];

@@ -38,6 +38,15 @@ struct RowCfg {
   static constexpr int LDS = ShapeInfo<N>::NSTEPS > 1 ? L * PITCH : 1;
 };
 
+// A cube of 1 GiB (512^3) is read and written past the 256 MiB memory-side cache:
+// its natural-order points and its spectrum are loaded and stored non-temporally,
+// which leaves that cache to the z-blocked slabs and is also faster by itself.  One
+// convolution in slabs: 2091 us with H and the y^-1 output streamed, 1995 with the
+// y input too, 1969 with the x^-1 pass, 1955 with the x pass (2153 with H
+// cached, 2344 with the y^-1 output cached, 2220 in whole-cube passes);
+// transforms 1315 -> 1225 forward, 1353 -> 1241 inverse.
+constexpr bool streamed(int n) { return n >= 512; }
+
 // x-axis pass; SCALE multiplies the result by `scale` (last inverse pass).
 template <int N, bool INV, bool SCALE>
 struct RowPass {
@@ -60,13 +69,13 @@ struct RowPass {
   __device__ __forceinline__ void load(int tile, Regs& r) const {
     const float2* src = in + base(tile);
 #pragma unroll
-    for (int m = 0; m < P; ++m) r.v[m] = src[T * m];
+    for (int m = 0; m < P; ++m) r.v[m] = ld_stream<streamed(N)>(src + T * m);
   }
   __device__ __forceinline__ void process(int tile, Regs& r) const {
     fft_line<N, INV, true>(r.v, t, RowLds{lds + l * K::PITCH}, tw_s);  // a row: lanes of one wave
     float2* dst = out + base(tile);
 #pragma unroll
-    for (int m = 0; m < P; ++m) dst[T * m] = SCALE ? cscale(r.v[m], scale) : r.v[m];
+    for (int m = 0; m < P; ++m) st_stream<streamed(N)>(dst + T * m, SCALE ? cscale(r.v[m], scale) : r.v[m]);
   }
 };
 
@@ -91,13 +100,17 @@ struct ColAddr {
 
 // y (AXIS 1) or z (AXIS 2) pass.  MODE 0 forward, 1 inverse, 2 forward * H
 // then inverse (z only).  IN_ZB / OUT_ZB: the input / output (and, for MODE 2,
-// the spectrum, which shares the output layout) are z-blocked.
-template <int N, int AXIS, int MODE, bool IN_ZB = false, bool OUT_ZB = false>
+// the spectrum, which shares the output layout) are z-blocked.  XG: the x groups
+// (of C columns) a launch covers, from the one that in, out and H point to: all
+// of a cube's, or a slab of them, whose z-blocked side is a buffer of the slab's
+// size that the next launch finds in the memory-side cache.
+template <int N, int AXIS, int MODE, bool IN_ZB = false, bool OUT_ZB = false, int XG = N / ColCfg<N>::C>
 struct ColPass {
   using K = ColCfg<N>;
   using AI = ColAddr<N, AXIS, IN_ZB>;
   using AO = ColAddr<N, AXIS, OUT_ZB>;
   static constexpr int P = K::P, T = K::T, C = K::C, G = K::G;
+  static constexpr int TILES = XG * (N / G);
   struct Regs {
     float2 v[P];
   };
@@ -111,32 +124,32 @@ struct ColPass {
 
   template <class A>
   __device__ __forceinline__ int offset(int tt) const {
-    const int xg = tt % (N / C);
-    const int other = (tt / (N / C)) * G + g;  // z for the y pass, y for the z pass
+    const int xg = tt % XG;
+    const int other = (tt / XG) * G + g;  // z for the y pass, y for the z pass
     return A::base(xg, c, other) + t * A::S;
   }
   __device__ __forceinline__ void load(int tile, Regs& r) const {
-    const int cube = tile / K::TILES, tt = tile % K::TILES;
+    const int cube = tile / TILES, tt = tile % TILES;
     const float2* src = in + (size_t)cube * N * N * N + offset<AI>(tt);
 #pragma unroll
-    for (int m = 0; m < P; ++m) r.v[m] = src[T * AI::S * m];
+    for (int m = 0; m < P; ++m) r.v[m] = ld_stream<streamed(N) && !IN_ZB>(src + T * AI::S * m);
   }
   __device__ __forceinline__ void process(int tile, Regs& r) const {
-    const int cube = tile / K::TILES, tt = tile % K::TILES;
+    const int cube = tile / TILES, tt = tile % TILES;
     const int off = offset<AO>(tt);
     const ColLds<C> view{lds + g * N * (C + 1) + c};
     if constexpr (MODE == 2) {
       fft_line<N, false>(r.v, t, view, tw_s);
       const float2* hp = H + (size_t)cube * hstride + off;
 #pragma unroll
-      for (int m = 0; m < P; ++m) r.v[m] = cmul(r.v[m], hp[T * AO::S * m]);
+      for (int m = 0; m < P; ++m) r.v[m] = cmul(r.v[m], ld_stream<streamed(N)>(hp + T * AO::S * m));
       fft_line<N, true>(r.v, t, view, tw_s);
     } else {
       fft_line<N, MODE == 1>(r.v, t, view, tw_s);
     }
     float2* dst = out + (size_t)cube * N * N * N + off;
 #pragma unroll
-    for (int m = 0; m < P; ++m) dst[T * AO::S * m] = r.v[m];
+    for (int m = 0; m < P; ++m) st_stream<streamed(N) && !OUT_ZB>(dst + T * AO::S * m, r.v[m]);
   }
 };
 
@@ -149,14 +162,14 @@ __device__ __forceinline__ void row_kernel(const float2* in, float2* out, const 
   run_tiles<N, K::THREADS>(k, ntotal, tw_s, tw);
 }
 
-template <int N, int AXIS, int MODE, bool IN_ZB = false, bool OUT_ZB = false>
+template <int N, int AXIS, int MODE, bool IN_ZB = false, bool OUT_ZB = false, int XG = N / ColCfg<N>::C>
 __device__ __forceinline__ void col_kernel(const float2* in, float2* out, const float2* H, const float2* tw,
                                            long long hstride, int ntotal) {
   using K = ColCfg<N>;
   __shared__ float2 lds[K::LDS];
   __shared__ float2 tw_s[N];
   const int c = threadIdx.x % K::C, t = (threadIdx.x / K::C) % K::T, g = threadIdx.x / (K::C * K::T);
-  const ColPass<N, AXIS, MODE, IN_ZB, OUT_ZB> k{in, out, H, tw_s, lds, hstride, c, t, g};
+  const ColPass<N, AXIS, MODE, IN_ZB, OUT_ZB, XG> k{in, out, H, tw_s, lds, hstride, c, t, g};
   run_tiles<N, K::THREADS>(k, ntotal, tw_s, tw);
 }
 

@@ -41,10 +41,25 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
   return make_float2(fmaf(a.x, b.x, -a.y * b.y), fmaf(a.x, b.y, a.y * b.x));
 }
 
-// load marked non-temporal (read once: it should not displace data that is
-// read again, such as a pass's intermediate kept in the MALL)
+// Loads and stores marked non-temporal: data that passes by once should not
+// displace what is read again, such as a pass's intermediate kept in the MALL.
+// (A two-float vector: through double the compiler drops the mark from stores.)
+typedef float f2_t __attribute__((ext_vector_type(2)));
+template <bool STREAM = true>
 __device__ __forceinline__ float2 ld_stream(const float2* p) {
-  return __builtin_bit_cast(float2, __builtin_nontemporal_load(reinterpret_cast<const double*>(p)));
+  if constexpr (STREAM) {
+    const f2_t v = __builtin_nontemporal_load(reinterpret_cast<const f2_t*>(p));
+    return make_float2(v.x, v.y);
+  } else {
+    return *p;
+  }
+}
+template <bool STREAM = true>
+__device__ __forceinline__ void st_stream(float2* p, float2 v) {
+  if constexpr (STREAM)
+    __builtin_nontemporal_store(f2_t{v.x, v.y}, reinterpret_cast<f2_t*>(p));
+  else
+    *p = v;
 }
 
 // Buffer accesses of one cube (at most 2^31 bytes): a per-thread 32-bit byte

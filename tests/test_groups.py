@@ -169,3 +169,39 @@ def test_graph_pair_keeps_order(gpu, overlap):
     batch.check()
     assert _same(buf, ref)
     batch.close()
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+def test_slabs_equal_axis_passes(gpu, in_place):
+    """One 512^3 convolution runs its y and z passes by slabs of x (conv_passes,
+    engine.cpp): the bits of the plan with whole-cube passes in natural order, and
+    five passes with the cube's own bytes in a timed call."""
+    import torch
+    api = gpu.api
+    n = 512
+    print("case slabs N=%d in_place=%s" % (n, in_place), flush=True)
+    sig = torch.empty(n ** 3, dtype=torch.complex64, device="cuda")
+    filt = torch.empty_like(sig)
+    api.fill_uniform(sig, 2 * sig.numel(), 67001)
+    api.fill_uniform(filt, 2 * filt.numel(), 67002)
+    ref = torch.empty_like(sig)
+    try:
+        api.set_plan(n, api.CF_PLAN_AXIS5)
+        natural = gpu.Spectrum(n, filt)
+        gpu.conv3d_device(natural, sig, ref)
+        natural.close()
+        api.set_plan(n, api.CF_PLAN_AXIS5Z)
+        spec = gpu.Spectrum(n, filt)
+    finally:
+        api.set_plan(n, api.CF_PLAN_AUTO)
+    out = sig.clone() if in_place else torch.zeros_like(sig)
+    gpu.conv3d_device(spec, out if in_place else sig, out)
+    assert _same(out, ref)
+    if not in_place:
+        out.zero_()
+        passes = gpu.conv3d_device_timed(spec, sig, out)
+        assert _same(out, ref)
+        assert [p["name"] for p in passes] == ["x_fwd", "y_fwd", "z_fwd_mul_z_inv", "y_inv", "x_inv"]
+        assert [p["bytes"] for p in passes] == [k * 8 * n ** 3 for k in (2, 2, 3, 2, 2)]
+        assert all(p["ms"] > 0 for p in passes)
+    spec.close()
