@@ -227,7 +227,7 @@ struct Xy1Pass {
   float scale;
   int rt, row, ry1, ry2l;  // row identity: row = y2l*16 + y1, thread t holds x = t + T*m
   int ckx, cy2l;           // column identity: (x, y2l) with x%GB fastest, then y2l, then x/GB
-  bool nt;                 // one cube per launch: signal read and output written non-temporally
+  bool nt;                 // one cube per launch: signal read (N = 256) and output written non-temporally
 
   __device__ __forceinline__ void tile_pos(int tile, size_t& cube, int& z, int& y2_0) const {
     cube = (size_t)(tile / K::A_TILES) * N * N * N;
@@ -425,7 +425,10 @@ __device__ __forceinline__ void xy1_kernel(const float2* in, float2* out, const 
   // signal and spectrum, read once, are loaded non-temporally (measured at
   // 256^3: 178 against 186 us per convolution); a launch over several cubes
   // is about 1% slower that way, so it keeps ordinary loads.
-  const bool nt = ntotal <= K::A_TILES;
+  // At 128^3 nothing of a convolution leaves the MALL and only the output is
+  // marked: a signal or spectrum still there from its writer is read from it
+  // (29.3 -> 27.9 us on buffers used again, 29.7 -> 29.2 on others).
+  const bool nt = ntotal <= K::A_TILES && (N >= 256 || INV);
   const P k{in, out, tw_s, lds, scale, x % K::T, row, row % 16, row / 16, cxh * GB + cxl, cy2l, nt};
   const int tile = xcd_group_tile<S>((int)blockIdx.x);
   typename P::Regs a;
@@ -491,7 +494,7 @@ struct MidPass {
   long long hstride;
   int l, zt;  // z-line identity: line l = y2*GM + x%GM, thread zt holds z = zt + T*m
   int q;      // first (kz, x%GM) row of the y2 transform: rows q + THREADS*rr, row = kz*GM + x%GM
-  bool nt;    // one cube per launch: its spectrum is read non-temporally
+  bool nt;    // one 256^3 cube per launch: its spectrum is read non-temporally
 
   // Buffer accesses (a 32-bit offset per thread, the strides of the loops in
   // the scalar offset) instead of a 64-bit address per access.
@@ -613,7 +616,7 @@ __device__ __forceinline__ void mid_kernel(const float2* in, float2* out, const 
   __shared__ float2 lds[M::LDS];
   __shared__ float2 tw_s[N];
   const int x = threadIdx.x;
-  const P k{in, out, H, tw_s, lds, hstride, x % M::LINES, x / M::LINES, x, ntotal <= M::TILES};
+  const P k{in, out, H, tw_s, lds, hstride, x % M::LINES, x / M::LINES, x, N >= 256 && ntotal <= M::TILES};
   // siblings (consecutive tiles of one x group) on one XCD, back to back
   const int tile = xcd_group_tile<M::SIBLINGS>((int)blockIdx.x);
   typename P::Regs a;
