@@ -566,7 +566,7 @@ void inv_passes(const SizeFns& f, unsigned n, unsigned nb, const void* in, void*
 // Small cubes have other forms of the same transforms (same bits): AXIS5 at N = 8
 // and 16 one pass over whole cubes, PLANE3 for one 64^3 cube smaller tiles with y
 // split over the passes, AXIS5Z for one 512^3 cube the y and z passes by slabs of
-// x.  own_passes: the plan's own passes in any case, for
+// x, G28M4 for several 128^3 cubes narrower tiles.  own_passes: the plan's own passes in any case, for
 // callers that report its forward and inverse half, or its tiles, by themselves.
 // Returns the index of the first pass after the product (the fpga_t split).
 size_t conv_passes(const SizeFns& f, int plan, unsigned n, unsigned nb, const void* sig, void* out, void* work,
@@ -621,7 +621,12 @@ size_t conv_passes(const SizeFns& f, int plan, unsigned n, unsigned nb, const vo
     return split;
   }
   if (is_split(plan)) {
-    const int vi = split_variant(plan);
+    // G28M4's wide outer tiles pay for one 128^3 cube, whose passes are one round of
+    // work-groups; batches run the passes of G24, which read the same spectrum (own
+    // filters, us per call, G28M4 / G24: 1 cube 28.1 / 29.4, 2 50.3 / 48.9, 4 86.3 /
+    // 84.1, 8 161 / 155, 40 811 / 783)
+    const bool narrow = plan == CF_PLAN_SPLIT3_G28M4 && n == 128 && nb > 1 && !own_passes;
+    const int vi = split_variant(narrow ? CF_PLAN_SPLIT3_G24 : plan);
     const unsigned at = cfgeo::split_a_threads((int)n, vi), aT = cfgeo::split_a_tiles((int)n, vi);
     const unsigned bt = cfgeo::split_b_threads((int)n, vi), bT = cfgeo::split_b_tiles((int)n, vi);
     const unsigned ct3 = cfgeo::split_c_threads((int)n, vi), cT3 = cfgeo::split_c_tiles((int)n, vi);
@@ -727,25 +732,31 @@ int run_passes(const PassList& v, unsigned n, unsigned nb, hipStream_t s, const 
 }
 
 // How many of `count` cubes of edge n go through a schedule's passes together:
-// groups of about kGroupBytes of cubes, evenly sized.  The next pass then finds
-// what a pass wrote in the 256 MiB memory-side cache.  Passes over the whole
-// batch against groups (us per call; one group when the batch holds fewer than
-// two of them): 4 x 256^3 own filters 752 -> 648, split-FP16 920 -> 812; 40 x
-// 128^3 824 -> 786 in groups of 8 (854 in groups of 4, whose passes no longer
-// fill the GPU; 822 in groups of 10); 300 x 64^3 721 -> 637 in groups of 64
-// (783 of 16); 4 transforms of 256^3 651 -> 535.
+// evenly sized groups of at most about kGroupBytes of cubes.  The next pass then
+// finds what a pass wrote in the 256 MiB memory-side cache.  Passes over the whole
+// batch against groups (us per call): 4 x 256^3 own filters 752 -> 648, split-FP16
+// 920 -> 812; 40 x 128^3 824 -> 786 in groups of 8 (854 in groups of 4, whose passes
+// no longer fill the GPU); 300 x 64^3 721 -> 637 in groups of 75 (783 of 16); 4
+// transforms of 256^3 651 -> 535.  A group may be larger by `slack` eighths, where
+// two smaller ones gain less from the cache than they lose (us per cube): 64^3 own
+// filters 40: 2.42, 64: 2.36, 72: 2.38, 80: 2.52, 127: 2.68, shared 40: 2.15, 64: 2.08,
+// 88: 2.08, 96: 2.13, transforms 40: 1.44, 88: 1.42, 127: 1.57; 128^3 own 5: 20.5, 8:
+// 19.5, 9: 22.0, 15: 26.8, shared 5: 19.6, 8: 19.0, 9: 19.3, 10: 20.1, 15: 22.8.
 constexpr size_t kGroupBytes = size_t(128) << 20;
-unsigned pass_group(unsigned n, unsigned count) {
-  const unsigned per = (unsigned)std::max<size_t>(1, kGroupBytes / cube_bytes(n));
-  const unsigned groups = std::max(1u, count / per);
+constexpr unsigned kTransformSlack = 3;
+unsigned conv_slack(int plan, bool own) { return needs_work(plan) ? (own ? 0 : 1) : (own ? 1 : 3); }
+unsigned pass_group(unsigned n, unsigned count, unsigned slack) {
+  const size_t per = std::max<size_t>(1, kGroupBytes / cube_bytes(n));
+  const unsigned most = (unsigned)(per + per * slack / 8);
+  const unsigned groups = count / most + (count % most != 0);
   return count / groups + (count % groups != 0);
 }
 
 // The convolution passes over how_many cubes, group by group.  work holds the
-// intermediates of one group (work_bytes of pass_group(n, how_many) cubes).
+// intermediates of one group (work_bytes of pass_group(...) cubes).
 int run_conv(const SizeFns& f, int plan, unsigned n, unsigned how_many, const void* sig, void* out, void* work,
              const void* H, long long hstride, float scale, int precision, hipStream_t s) {
-  const unsigned group = pass_group(n, how_many);
+  const unsigned group = pass_group(n, how_many, conv_slack(plan, hstride != 0));
   const size_t V = cube_bytes(n);
   for (unsigned b = 0; b < how_many; b += group) {
     const unsigned nb = std::min(group, how_many - b);
@@ -1619,7 +1630,7 @@ extern "C" int cf_spectrum_create(unsigned n, unsigned count, const void* filter
   int rc = e == hipSuccess ? choose_plan(n, f, &h->plan)
                            : fail(CF_ERR_RUNTIME, "hipMemcpyAsync: %s", hipGetErrorString(e));
   void* work = nullptr;
-  const unsigned group = pass_group(n, count);
+  const unsigned group = pass_group(n, count, needs_work(h->plan) ? 1 : kTransformSlack);
   if (rc == CF_OK && needs_work(h->plan)) rc = acquire_work(cube_bytes(n) * group, s, &work);
   for (unsigned b = 0; b < count && rc == CF_OK; b += group) {
     const unsigned nb = std::min(group, count - b);
@@ -1735,7 +1746,7 @@ static int conv_device_impl(cf_spectrum_t h, const void* d_sig, void* d_out, uns
   const long long hstride = h->count == 1 ? 0 : (long long)cube_elems(n);
   hipStream_t s = (hipStream_t)stream;
   h->mem->use(s);
-  const unsigned group = pass_group(n, how_many);
+  const unsigned group = pass_group(n, how_many, conv_slack(h->plan, hstride != 0));
   void* work = nullptr;
   if (needs_work(h->plan)) CFCHK(acquire_work(work_bytes(h->plan, n, group, d_sig, d_out), s, &work));
   struct WorkRelease {  // the workspace is marked busy on s whatever path returns
@@ -1981,7 +1992,7 @@ extern "C" int cf_fft3d_device(unsigned n, const void* d_in, void* d_out, unsign
   SizeFns* f = nullptr;
   CFCHK(size_res(n, &f));
   hipStream_t s = (hipStream_t)stream;
-  const unsigned group = pass_group(n, how_many);
+  const unsigned group = pass_group(n, how_many, kTransformSlack);
   // 256^3 in two passes through the workspace (97 us against 133 forward, 143
   // inverse in one pass per axis).  A call recorded into a graph would share
   // the workspace with whatever runs beside its replays, and cannot allocate
@@ -2417,8 +2428,9 @@ static int batch_create(const cf_instance_t* inst, unsigned count, int scale_mod
              (const char*)inst[i + run].d_sig == (const char*)inst[i].d_sig + run * V &&
              (char*)inst[i + run].d_out == (char*)inst[i].d_out + run * V)
         ++run;
-      work_need = std::max(work_need, work_bytes(inst[i].h->plan, n, pass_group(n, run), inst[i].d_sig,
-                                                 inst[i].d_out));
+      const int plan = inst[i].h->plan;
+      work_need = std::max(work_need, work_bytes(plan, n, pass_group(n, run, conv_slack(plan, run > 1 && !shared)),
+                                                 inst[i].d_sig, inst[i].d_out));
       runs.push_back({i, run, shared});
       i += run;
     }
@@ -2438,7 +2450,7 @@ static int batch_create(const cf_instance_t* inst, unsigned count, int scale_mod
     };
     // a 64^3 and a 32^3 run next to each other go through the plane plan's passes
     // together (plane_pair.h), if neither writes what the other reads or writes, so
-    // that their order does not show, and each is one group of run_conv.  Three
+    // that their order does not show, and neither is more than a group.  Three
     // launches are saved whatever the counts: 8 + 16 cubes 37.7 us against 36.0 +
     // 19.9 as graphs of their own (53.3 with an 8^3 instance between the two that
     // keeps them apart), 1 + 1 19.3 against 30.2, 64 + 128 190 against 201.
@@ -2447,7 +2459,7 @@ static int batch_create(const cf_instance_t* inst, unsigned count, int scale_mod
       if (!(a.h->n == 64 && c.h->n == 32) && !(a.h->n == 32 && c.h->n == 64)) return false;
       if (a.h->plan != CF_PLAN_PLANE3 || c.h->plan != CF_PLAN_PLANE3) return false;
       const size_t na = cube_bytes(a.h->n) * x.run, nc = cube_bytes(c.h->n) * y.run;
-      if (pass_group(a.h->n, x.run) < x.run || pass_group(c.h->n, y.run) < y.run) return false;
+      if (na > kGroupBytes || nc > kGroupBytes) return false;
       auto meet = [](const void* p, size_t np, const void* q, size_t nq) {
         return (const char*)p < (const char*)q + nq && (const char*)q < (const char*)p + np;
       };

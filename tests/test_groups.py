@@ -12,8 +12,10 @@ def _same(a, b):
     return torch.equal(torch.view_as_real(a).view(torch.int32), torch.view_as_real(b).view(torch.int32))
 
 
-# 128 MiB of cubes make a group: 8 at 128^3, 64 at 64^3, 1 at 256^3
-@pytest.mark.parametrize("n,count", [(128, 15), (128, 17), (64, 130), (256, 2), (256, 3)])
+# the largest groups: 8 (own filters) and 9 (one filter) cubes of 128^3, 72 and 88 of
+# 64^3, 1 of 256^3
+@pytest.mark.parametrize("n,count", [(128, 9), (128, 10), (128, 15), (128, 17), (64, 73), (64, 89), (64, 130), (256, 2),
+                                     (256, 3)])
 @pytest.mark.parametrize("in_place", [False, True])
 def test_groups_equal_single_cubes(gpu, n, count, in_place):
     import torch
@@ -205,3 +207,36 @@ def test_slabs_equal_axis_passes(gpu, in_place):
         assert [p["bytes"] for p in passes] == [k * 8 * n ** 3 for k in (2, 2, 3, 2, 2)]
         assert all(p["ms"] > 0 for p in passes)
     spec.close()
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("n", [128, 256])
+def test_batches_of_the_wide_plan(gpu, n, in_place):
+    """A batch of 128^3 cubes with a spectrum of split3_g28m4 runs the passes of
+    split3_g24 (conv_passes, engine.cpp), a single cube its own: the bits of single
+    cubes, and of 256^3 batches, which keep them."""
+    import torch
+    api = gpu.api
+    count = 3
+    print("case wide plan N=%d in_place=%s" % (n, in_place), flush=True)
+    sig = torch.empty((count, n ** 3), dtype=torch.complex64, device="cuda")
+    filt = torch.empty_like(sig)
+    api.fill_uniform(sig, 2 * sig.numel(), 68000 + n)
+    api.fill_uniform(filt, 2 * filt.numel(), 69000 + n)
+    try:
+        api.set_plan(n, api.CF_PLAN_SPLIT3_G28M4)
+        spec, shared = gpu.Spectrum(n, filt, count), gpu.Spectrum(n, filt)
+        singles = [gpu.Spectrum(n, filt[k]) for k in range(count)]
+    finally:
+        api.set_plan(n, api.CF_PLAN_AUTO)
+    want = torch.empty_like(sig)
+    want_sh = torch.empty_like(sig)
+    for k in range(count):
+        gpu.conv3d_device(singles[k], sig[k], want[k])
+        gpu.conv3d_device(shared, sig[k], want_sh[k])
+    for h, ref in ((spec, want), (shared, want_sh)):
+        out = sig.clone() if in_place else torch.empty_like(sig)
+        gpu.conv3d_device(h, out if in_place else sig, out, count)
+        assert _same(out, ref)
+    for h in [spec, shared] + singles:
+        h.close()
