@@ -69,7 +69,9 @@ struct SizeFns {
   hipFunction_t cube_fwd = nullptr, cube_inv = nullptr, cube_conv = nullptr;  // N in {8, 16}: a cube per work-group
   hipFunction_t plane_fwd = nullptr, plane_inv = nullptr;                 // N in {32, 64, 128}
   hipFunction_t rows_fwd = nullptr, rows_inv = nullptr, mid_split = nullptr;  // N = 64, one cube of the plane plan
-  hipFunction_t coly_fwd_slab = nullptr, colz_conv_slab = nullptr, coly_inv_slab = nullptr;  // N = 512, by x slabs
+  // N = 512, by x slabs
+  hipFunction_t coly_fwd_slab = nullptr, colz_conv_slab = nullptr, coly_inv_slab = nullptr;
+  hipFunction_t colz_fwd_slab = nullptr, colz_inv_slab = nullptr;
   hipFunction_t coly_fwd_zb = nullptr, coly_inv_zb = nullptr, colz_fwd_zb = nullptr, colz_conv_zb = nullptr;  // N >= 64
   hipFunction_t xy1_fwd[cfgeo::kSplitVariants] = {}, xy1_inv[cfgeo::kSplitVariants] = {};  // N = 256
   hipFunction_t mid[cfgeo::kSplitVariants] = {}, mspec[cfgeo::kSplitVariants] = {};
@@ -439,6 +441,8 @@ int size_res(unsigned n, SizeFns** out) {
     CFCHK(get_fn(&s.coly_fwd_slab, "cf_coly_fwd_slab_512"));
     CFCHK(get_fn(&s.colz_conv_slab, "cf_colz_conv_slab_512"));
     CFCHK(get_fn(&s.coly_inv_slab, "cf_coly_inv_slab_512"));
+    CFCHK(get_fn(&s.colz_fwd_slab, "cf_colz_fwd_slab_512"));
+    CFCHK(get_fn(&s.colz_inv_slab, "cf_colz_inv_slab_512"));
     CFCHK(get_fn(&s.mx_coly_fwd_zb, "cf_coly_fwd_zb_512_s"));
     CFCHK(get_fn(&s.mx_colz_conv_zb, "cf_colz_conv_zb_512_s"));
     CFCHK(get_fn(&s.mx_coly_inv_zb, "cf_coly_inv_zb_512_s"));
@@ -719,6 +723,37 @@ void spectrum_passes(const SizeFns& f, int plan, unsigned n, unsigned count, con
   const unsigned bt = cfgeo::split_b_threads((int)n, vi), bT = cfgeo::split_b_tiles((int)n, vi);
   v.push_back({f.xy1_fwd[vi], aT, at, src, work, nullptr, 0, 1.0f, "xy1_fwd", io});
   v.push_back({f.mspec[vi], bT, bt, work, dst, nullptr, 0, 1.0f, "y2z_fwd", io});
+}
+
+// A transform through a workspace (fft_work_bytes): 256^3 in two passes, 512^3 with
+// its y and z passes by x slabs.
+size_t fft_work_bytes(unsigned n, unsigned nb) {
+  return n == 256 ? cube_bytes(n) * nb : n == 512 ? (size_t)cfgeo::slab_bytes : 0;
+}
+void fft_work_passes(const SizeFns& f, unsigned n, unsigned nb, const void* in, void* out, void* work, bool inverse,
+                     PassList& v) {
+  const double io = 2.0 * cube_bytes(n) * nb;
+  if (n == 256) {
+    const int d = inverse ? 1 : 0;
+    v.push_back({f.fft2_first[d], cfgeo::fft2_first_tiles, cfgeo::fft2_first_threads, in, work, nullptr, 0, 1.0f, "yz1", io});
+    v.push_back({f.fft2_second[d], cfgeo::fft2_second_tiles, cfgeo::fft2_second_threads, work, out, nullptr, 0, 1.0f, "z2x", io});
+    return;
+  }
+  const unsigned rt = cfgeo::row_threads(n), rT = cfgeo::row_tiles(n), ct = cfgeo::col_threads(n), sT = cfgeo::slab_tiles;
+  const double sio = io / cfgeo::slabs_512;
+  if (!inverse) v.push_back({f.row_fwd, rT, rt, in, out, nullptr, 0, 1.0f, "x_fwd", io});
+  for (unsigned k = 0; k < (unsigned)cfgeo::slabs_512; ++k) {
+    const size_t x = (size_t)k * cfgeo::slab_groups * cfgeo::col_c(512) * 8;
+    char* o = (char*)out + x;
+    if (inverse) {
+      v.push_part({f.colz_inv_slab, sT, ct, (const char*)in + x, work, nullptr, 0, 1.0f, "z_inv", sio}, 0);
+      v.push_part({f.coly_inv_slab, sT, ct, work, o, nullptr, 0, 1.0f, "y_inv", sio}, 1);
+    } else {
+      v.push_part({f.coly_fwd_slab, sT, ct, o, work, nullptr, 0, 1.0f, "y_fwd", sio}, 1);
+      v.push_part({f.colz_fwd_slab, sT, ct, work, o, nullptr, 0, 1.0f, "z_fwd", sio}, 2);
+    }
+  }
+  if (inverse) v.push_back({f.row_inv, rT, rt, out, out, nullptr, 0, 1.0f, "x_inv", io});
 }
 
 int run_passes(const PassList& v, unsigned n, unsigned nb, hipStream_t s, const void* tw,
@@ -1994,15 +2029,15 @@ extern "C" int cf_fft3d_device(unsigned n, const void* d_in, void* d_out, unsign
   hipStream_t s = (hipStream_t)stream;
   const unsigned group = pass_group(n, how_many, kTransformSlack);
   // 256^3 in two passes through the workspace (97 us against 133 forward, 143
-  // inverse in one pass per axis).  A call recorded into a graph would share
-  // the workspace with whatever runs beside its replays, and cannot allocate
-  // it: it keeps the axis passes, as does a call that finds no memory for it.
+  // inverse in one pass per axis), 512^3 by slabs (1073 against 1230 forward, 1157
+  // against 1245 inverse).  A call recorded into a graph would share the workspace
+  // with whatever runs beside its replays, and cannot allocate it: it keeps the axis
+  // passes, as does a call that finds no memory for it.
   void* work = nullptr;
-  if (n == 256) {
-    if (!capturing(s) && acquire_work(g.fft_work, cube_bytes(n) * group, s, &work) != CF_OK) {
-      (void)hipGetLastError();
-      work = nullptr;
-    }
+  const size_t need = fft_work_bytes(n, group);
+  if (need && !capturing(s) && acquire_work(g.fft_work, need, s, &work) != CF_OK) {
+    (void)hipGetLastError();
+    work = nullptr;
   }
   struct WorkRelease {
     void* w;
@@ -2016,12 +2051,9 @@ extern "C" int cf_fft3d_device(unsigned n, const void* d_in, void* d_out, unsign
     const void* in = (const char*)d_in + b * cube_bytes(n);
     void* out = (char*)d_out + b * cube_bytes(n);
     PassList p;
-    if (work) {
-      const double io = 2.0 * cube_bytes(n) * nb;
-      const int d = inverse ? 1 : 0;
-      p.push_back({f->fft2_first[d], cfgeo::fft2_first_tiles, cfgeo::fft2_first_threads, in, work, nullptr, 0, 1.0f, "yz1", io});
-      p.push_back({f->fft2_second[d], cfgeo::fft2_second_tiles, cfgeo::fft2_second_threads, work, out, nullptr, 0, 1.0f, "z2x", io});
-    } else if (inverse)
+    if (work)
+      fft_work_passes(*f, n, nb, in, out, work, inverse != 0, p);
+    else if (inverse)
       inv_passes(*f, n, nb, in, out, 1.0f, p);
     else
       fwd_passes(*f, n, nb, in, out, p);

@@ -32,6 +32,7 @@ constexpr bool supported(int n) { return points_per_thread(n) != 0; }
 // slabs of 2: 2278 us, 4: 2050, 8: 1956, 16: 2303)
 constexpr int slab_groups = 8, slabs_512 = 512 / col_c(512) / slab_groups;
 constexpr int slab_tiles = slab_groups * (512 / col_g(512));
+constexpr unsigned long long slab_bytes = 8ull * slab_groups * col_c(512) * 512 * 512;
 
 // a whole cube per work-group, one line of n points per thread (n*n threads)
 constexpr bool cube_supported(int n) { return n == 8 || n == 16; }

@@ -83,7 +83,7 @@ CF_INSTANTIATE(128)
 CF_INSTANTIATE(256)
 CF_INSTANTIATE(512)
 
-// y, z * H * z^-1 and y^-1 of 512^3 by x slabs
+// y, z * H * z^-1 and y^-1 of 512^3 by x slabs, and z and z^-1 of its transforms
 extern "C" __global__ __launch_bounds__(cfk::ColCfg<512>::THREADS) void cf_coly_fwd_slab_512(CF_ARGS) {
   cfk::col_kernel<512, 1, 0, false, true, cfgeo::slab_groups>(in, out, H, tw, hstride, ntotal);
 }
@@ -92,6 +92,12 @@ extern "C" __global__ __launch_bounds__(cfk::ColCfg<512>::THREADS) void cf_colz_
 }
 extern "C" __global__ __launch_bounds__(cfk::ColCfg<512>::THREADS) void cf_coly_inv_slab_512(CF_ARGS) {
   cfk::col_kernel<512, 1, 1, true, false, cfgeo::slab_groups>(in, out, H, tw, hstride, ntotal);
+}
+extern "C" __global__ __launch_bounds__(cfk::ColCfg<512>::THREADS) void cf_colz_fwd_slab_512(CF_ARGS) {
+  cfk::col_kernel<512, 2, 0, true, false, cfgeo::slab_groups>(in, out, H, tw, hstride, ntotal);
+}
+extern "C" __global__ __launch_bounds__(cfk::ColCfg<512>::THREADS) void cf_colz_inv_slab_512(CF_ARGS) {
+  cfk::col_kernel<512, 2, 1, false, true, cfgeo::slab_groups>(in, out, H, tw, hstride, ntotal);
 }
 CF_INSTANTIATE_ZB(64)
 CF_INSTANTIATE_ZB(128)
