@@ -248,7 +248,6 @@ __device__ __forceinline__ void xy1_mfma_kernel(const float2* in, float2* out, c
   __shared__ float2 lds[X::LDS];
   __shared__ float2 tw_s[256], tw_a[256];
   __shared__ float red[X::WAVES];
-  stage_twiddles<256, X::THREADS>(tw_s, tw);
   const void* optab = tw + 256;  // DFT16 operand table follows the twiddles
   const int tile = xcd_group_tile<X::S>((int)blockIdx.x);
   if (tile >= ntotal) return;
@@ -273,6 +272,7 @@ __device__ __forceinline__ void xy1_mfma_kernel(const float2* in, float2* out, c
         im[4 * b + i] = t.y;
       }
     }
+    stage_twiddles<256, X::THREADS>(tw_s, tw);  // with the tile's loads in flight
     const int e = fp16_exp(block_max<X::WAVES>(absmax16(re, im), red));
     scale_soa(re, im, ldexpf(1.0f, e));
     scaled_table(tw_a, tw_s, ldexpf(1.0f, 12 - e));  // final twiddle and unscale (three stages of 1/16)
@@ -334,6 +334,7 @@ __device__ __forceinline__ void xy1_mfma_kernel(const float2* in, float2* out, c
         im[4 * b + i] = t.y;
       }
     }
+    stage_twiddles<256, X::THREADS>(tw_s, tw);
     const int e = fp16_exp(block_max<X::WAVES>(absmax16(re, im), red));
     scaled_table(tw_a, tw_s, ldexpf(1.0f, e));  // input scale, folded into the first twiddle
     __syncthreads();
@@ -423,7 +424,6 @@ __device__ __forceinline__ void mid_mfma_kernel(const float2* in, float2* out, c
   __shared__ float2 lds[Q::LDS];
   __shared__ float2 tw_s[256];
   __shared__ float red[2][Q::WAVES];
-  stage_twiddles<256, Q::THREADS>(tw_s, tw);
   const void* optab = tw + 256;  // DFT16 operand table follows the twiddles
   const int tile = xcd_group_tile<M::SIBLINGS>((int)blockIdx.x);
   if (tile >= ntotal) return;
@@ -437,6 +437,13 @@ __device__ __forceinline__ void mid_mfma_kernel(const float2* in, float2* out, c
   // this thread's point z = (4zq + b) + 16(4g + i) at voff + (b + 16 i) ZB
   const unsigned voff = (unsigned)K::mid_index(x0 + xl, k1, y2, 4 * zq + 64 * g) * (unsigned)sizeof(float2);
   const __amdgpu_buffer_rsrc_t rin = buffer_rsrc(in + cube, CUBE), rout = buffer_rsrc(out + cube, CUBE);
+  // The 64-byte operand row of each direction is read once, ahead of what it
+  // waits with (the tile's loads, the second maximum), and held in 16 VGPRs over
+  // its three stages (128 VGPRs, no spills).  Read again after each barrier, every
+  // stage began with the latency of a table that the tile's own loads push out of
+  // the L1.  Four convolutions with own filters: 803 us re-read, 757 each read
+  // ahead of the stage's exchange, 734 held.
+  const Dft16Ops fops = dft16_ops<false>(optab);
   float re[16], im[16];
 #pragma unroll
   for (int b = 0; b < 4; ++b)
@@ -446,6 +453,7 @@ __device__ __forceinline__ void mid_mfma_kernel(const float2* in, float2* out, c
       re[4 * b + i] = t.x;
       im[4 * b + i] = t.y;
     }
+  stage_twiddles<256, Q::THREADS>(tw_s, tw);  // with the tile's loads in flight
   // the spectrum values, loaded with the points (their latency hidden behind the forward half)
   float2 hreg[16];
   {
@@ -461,10 +469,8 @@ __device__ __forceinline__ void mid_mfma_kernel(const float2* in, float2* out, c
   }
   const int e1 = fp16_exp(block_max<Q::WAVES>(absmax16(re, im), red[0]));
   scale_soa(re, im, ldexpf(1.0f, e1));
-  // (the operand table is re-read before each stage rather than held in 16
-  // VGPRs across the pass: the kernel stays within 128 VGPRs without spills)
   // z: stage A over m for t = 4zq+b -> k0 = 4g+i, twiddle W256^(t k0)
-  dft16x4_mfma(re, im, dft16_ops<false>(optab));
+  dft16x4_mfma(re, im, fops);
 #pragma unroll
   for (int b = 0; b < 4; ++b)
 #pragma unroll
@@ -479,7 +485,7 @@ __device__ __forceinline__ void mid_mfma_kernel(const float2* in, float2* out, c
     for (int i = 0; i < 4; ++i)
       lds_get(lds, (4 * g + i) * Q::E_ZT + (4 * zq + b) * Q::E_K0 + line, re[4 * b + i], im[4 * b + i]);
   // stage B over t for k0 = 4zq+b -> k1' = 4g+i: kz = k0 + 16 k1'
-  dft16x4_mfma(re, im, dft16_ops<false>(optab));
+  dft16x4_mfma(re, im, fops);
   __syncthreads();  // E read everywhere before F overwrites it
 #pragma unroll
   for (int b = 0; b < 4; ++b)
@@ -494,15 +500,16 @@ __device__ __forceinline__ void mid_mfma_kernel(const float2* in, float2* out, c
 #pragma unroll
     for (int i = 0; i < 4; ++i) lds_get(lds, kz * Q::F_KZ + (4 * g + i) * GM + xb, re[4 * b + i], im[4 * b + i]);
   }
-  dft16x4_mfma(re, im, dft16_ops<false>(optab));
+  dft16x4_mfma(re, im, fops);
 #pragma unroll
   for (int b = 0; b < 4; ++b)
 #pragma unroll
     for (int i = 0; i < 4; ++i)  // H at k2 = 4g+i, column beta = 16(4w+b) + j
       cmul_soa(re[4 * b + i], im[4 * b + i], hreg[4 * b + i]);
+  const Dft16Ops iops = dft16_ops<true>(optab);
   const int e2 = fp16_exp(block_max<Q::WAVES>(absmax16(re, im), red[1]));  // also: F read everywhere
   scale_soa(re, im, ldexpf(1.0f, e2));
-  dft16x4_mfma(re, im, dft16_ops<true>(optab));  // -> y2 = 4g+i
+  dft16x4_mfma(re, im, iops);  // -> y2 = 4g+i
   // The inverse half recomputes the thread's indices from its id, kept opaque
   // to the compiler, rather than holding the forward half's values across
   // the pass (which made the kernel spill to scratch at 128 VGPRs).
@@ -524,7 +531,7 @@ __device__ __forceinline__ void mid_mfma_kernel(const float2* in, float2* out, c
     for (int i = 0; i < 4; ++i)
       lds_get(lds, (4 * zq2 + b + 16 * (4 * g2 + i)) * Q::F_KZ + line2, re[4 * b + i], im[4 * b + i]);
   // inverse z: stage A over m = k1' for t = k0 = 4zq+b -> q = 4g+i, twiddle conj W256^(t q)
-  dft16x4_mfma(re, im, dft16_ops<true>(optab));
+  dft16x4_mfma(re, im, iops);
   __syncthreads();  // F read everywhere before E overwrites it
 #pragma unroll
   for (int b = 0; b < 4; ++b)
@@ -540,7 +547,7 @@ __device__ __forceinline__ void mid_mfma_kernel(const float2* in, float2* out, c
     for (int i = 0; i < 4; ++i)
       lds_get(lds, (4 * g2 + i) * Q::E_ZT + (4 * zq2 + b) * Q::E_K0 + line2, re[4 * b + i], im[4 * b + i]);
   // stage B over t for q = 4zq+b -> r = 4g+i: z = q + 16 r; six stages of 1/16
-  dft16x4_mfma(re, im, dft16_ops<true>(optab));
+  dft16x4_mfma(re, im, iops);
   const float un = ldexpf(1.0f, 24 - e1 - e2);
 #pragma unroll
   for (int b = 0; b < 4; ++b)
