@@ -185,7 +185,7 @@ struct Engine {
   bool stage_used[2] = {false, false};
   size_t h_out_bytes = 0;
   Workspace work;      // of the plans that go through one
-  Workspace fft_work;  // of the two-pass plain transform; of its own, so that a transform
+  Workspace fft_work;  // of the plain 256^3 and 512^3 transforms; of its own, so that a transform
                        // meets neither the convolutions of other streams nor a graph
                        // that holds the address of theirs
   std::vector<SpecMem> spec_pool;
