@@ -2032,10 +2032,11 @@ extern "C" int cf_fft3d_device(unsigned n, const void* d_in, void* d_out, unsign
   // inverse in one pass per axis), 512^3 by slabs (1073 against 1230 forward, 1157
   // against 1245 inverse).  A call recorded into a graph would share the workspace
   // with whatever runs beside its replays, and cannot allocate it: it keeps the axis
-  // passes, as does a call that finds no memory for it.
+  // passes, as does a call that finds no memory for it, and one on hipStreamPerThread,
+  // a stream of its own in every thread under one handle, which nothing orders.
   void* work = nullptr;
   const size_t need = fft_work_bytes(n, group);
-  if (need && !capturing(s) && acquire_work(g.fft_work, need, s, &work) != CF_OK) {
+  if (need && s != hipStreamPerThread && !capturing(s) && acquire_work(g.fft_work, need, s, &work) != CF_OK) {
     (void)hipGetLastError();
     work = nullptr;
   }

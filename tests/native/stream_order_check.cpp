@@ -1,0 +1,69 @@
+// Order between the library's launches on several streams and threads, checked
+// on a recording HIP runtime (hip_recorder.h).  One check per run, named by the
+// argument; prints "ok" and exits 0 when it holds.
+#include <cstdio>
+#include <cstring>
+
+#include "convfpga/convfpga_ext.h"
+#include "hip_recorder.h"
+
+// (convfpga.h and the HIP headers both name a float2)
+extern "C" int fpga_initialize(const char*, const char*, bool);
+
+static int failures = 0;
+#define CHECK(c)                                            \
+  do {                                                      \
+    if (!(c)) {                                             \
+      printf("line %d: %s\n", __LINE__, #c);                \
+      ++failures;                                           \
+    }                                                       \
+  } while (0)
+
+static size_t cube(unsigned n) { return (size_t)n * n * n * 8; }
+static void forget() {
+  rec::launches.clear();
+  rec::faults.clear();
+  rec::device_waits = rec::captured_launches = 0;
+}
+struct Bufs {
+  char *in, *out;
+  explicit Bufs(unsigned n, unsigned count = 1) : in(rec::alloc(cube(n) * count)), out(rec::alloc(cube(n) * count)) {}
+};
+static int fft(unsigned n, const Bufs& b, hipStream_t s, int inverse = 0) {
+  return cf_fft3d_device(n, b.in, b.out, 1, inverse, s);
+}
+
+// Transforms on hipStreamPerThread, which is another stream in every thread: they
+// meet in no memory, and neither do one on it and one on a stream of another thread.
+static void fft_per_thread() {
+  for (unsigned n : {256u, 512u})
+    for (int inverse : {0, 1}) {
+      Bufs a(n), b(n), c(n);
+      fft(n, a, hipStreamPerThread, inverse);
+      forget();
+      std::thread([&] { CHECK(fft(n, a, hipStreamPerThread, inverse) == CF_OK); }).join();
+      std::thread([&] { CHECK(fft(n, b, hipStreamPerThread, inverse) == CF_OK); }).join();
+      CHECK(fft(n, c, rec::new_stream(), inverse) == CF_OK);
+      CHECK(rec::races() == 0);
+      CHECK(rec::faults.empty());
+    }
+}
+
+int main(int argc, char** argv) {
+  const struct {
+    const char* name;
+    void (*run)();
+  } checks[] = {{"fft_per_thread", fft_per_thread}};
+  CHECK(fpga_initialize("gfx950", "recorded", false) == 0);
+  bool found = false;
+  for (auto& c : checks)
+    if (argc == 2 && !strcmp(argv[1], c.name)) {
+      c.run();
+      found = true;
+    }
+  CHECK(found);
+  for (auto& f : rec::faults) printf("%s\n", f.c_str());
+  if (failures) return 1;
+  printf("ok %s\n", argv[1]);
+  return 0;
+}
