@@ -113,14 +113,18 @@ bool plan_ok(unsigned n, int plan) {
   return false;
 }
 
-// Device workspace shared by the calls of all streams, ordered by ev.
-struct Workspace {
-  void* d = nullptr;
-  size_t bytes = 0;
-  hipStream_t stream = nullptr;  // of the last user
-  bool used = false;
-  hipEvent_t ev = nullptr;
+// Device workspace of the plain 256^3 and 512^3 transforms of one stream.  Every
+// stream has its own, so that transforms on different streams stay independent
+// (no order between them, and no call on a stream that may be recording a graph)
+// and meet neither the convolutions' workspace nor a graph that holds the address
+// of that one.  At most kFftWorkStreams of them, for the streams that come first;
+// transforms on others run one pass per axis, as without a workspace.
+struct FftWork {
+  hipStream_t stream;
+  void* d;
 };
+constexpr size_t kFftWorkStreams = 4;
+constexpr size_t kFftWorkBytes = std::max<size_t>(cfgeo::slab_bytes, size_t(8) << 24);  // a 512^3 slab, a 256^3 cube
 
 // true if calls on s are being recorded into a graph (or that cannot be told)
 bool capturing(hipStream_t s) {
@@ -184,10 +188,13 @@ struct Engine {
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
   bool stage_used[2] = {false, false};
   size_t h_out_bytes = 0;
-  Workspace work;      // of the plans that go through one
-  Workspace fft_work;  // of the plain 256^3 and 512^3 transforms; of its own, so that a transform
-                       // meets neither the convolutions of other streams nor a graph
-                       // that holds the address of theirs
+  // workspace of the plans that go through one, ordered across streams by work_ev
+  void* d_work = nullptr;
+  size_t d_work_bytes = 0;
+  hipStream_t work_stream = nullptr;
+  bool work_used = false;
+  hipEvent_t work_ev = nullptr;
+  std::vector<FftWork> fft_work;
   std::vector<SpecMem> spec_pool;
   std::string arch;
   // error-norm scratch
@@ -259,11 +266,15 @@ void release_all() {
   if (g.d_data) (void)hipFree(g.d_data);
   if (g.d_filt) (void)hipFree(g.d_filt);
   if (g.d_err) (void)hipFree(g.d_err);
-  for (Workspace* w : {&g.work, &g.fft_work}) {
-    if (w->d) (void)hipFree(w->d);
-    if (w->ev) (void)hipEventDestroy(w->ev);
-    *w = Workspace();
-  }
+  if (g.d_work) (void)hipFree(g.d_work);
+  g.d_work = nullptr;
+  g.d_work_bytes = 0;
+  g.work_used = false;
+  g.work_stream = nullptr;
+  if (g.work_ev) (void)hipEventDestroy(g.work_ev);
+  g.work_ev = nullptr;
+  for (FftWork& w : g.fft_work) (void)hipFree(w.d);
+  g.fft_work.clear();
   if (g.h_sig) (void)hipHostFree(g.h_sig);
   if (g.h_filt) (void)hipHostFree(g.h_filt);
   if (g.h_out) (void)hipHostFree(g.h_out);
@@ -948,46 +959,63 @@ double host_ms(std::chrono::steady_clock::time_point a, std::chrono::steady_cloc
 }
 
 // Workspace of `bytes` for a call on stream s.  Calls on different streams are
-// ordered through w.ev so that they never overlap on it.
-int acquire_work(Workspace& w, size_t bytes, hipStream_t s, void** out) {
-  if (!w.ev) HIPCHK(hipEventCreateWithFlags(&w.ev, hipEventDisableTiming));
-  if (w.bytes < bytes) {
-    if (w.d) {
+// ordered through work_ev so that they never overlap on the shared workspace.
+int acquire_work(size_t bytes, hipStream_t s, void** out) {
+  if (!g.work_ev) HIPCHK(hipEventCreateWithFlags(&g.work_ev, hipEventDisableTiming));
+  if (g.d_work_bytes < bytes) {
+    if (g.d_work) {
       HIPCHK(hipDeviceSynchronize());  // earlier users on any stream are done
-      (void)hipFree(w.d);
+      (void)hipFree(g.d_work);
     }
-    w.d = nullptr;
-    w.bytes = 0;
-    w.used = false;
-    hipError_t e = dev_malloc(&w.d, bytes);
+    g.d_work = nullptr;
+    g.d_work_bytes = 0;
+    g.work_used = false;
+    hipError_t e = dev_malloc(&g.d_work, bytes);
     if (e != hipSuccess) return fail(CF_ERR_NOMEM, "hipMalloc(%zu) for the workspace: %s", bytes, hipGetErrorString(e));
-    w.bytes = bytes;
+    g.d_work_bytes = bytes;
   }
-  if (w.used && w.stream != s) {
+  if (g.work_used && g.work_stream != s) {
     // Everything submitted so far to the previous user's stream includes its
     // use of the workspace, so an event recorded there now orders s after it.
     // (Recording lazily, only on a change of stream, keeps event packets --
     // each a gap of several microseconds on the GPU -- out of the
     // single-stream sequence.)  A stream destroyed meanwhile has finished its
     // work; should the record fail, wait for the whole device instead.
-    if (hipEventRecord(w.ev, w.stream) == hipSuccess) {
-      HIPCHK(hipStreamWaitEvent(s, w.ev, 0));
+    if (hipEventRecord(g.work_ev, g.work_stream) == hipSuccess) {
+      HIPCHK(hipStreamWaitEvent(s, g.work_ev, 0));
     } else {
       (void)hipGetLastError();
       HIPCHK(hipDeviceSynchronize());
     }
   }
-  *out = w.d;
+  *out = g.d_work;
   return CF_OK;
 }
-int acquire_work(size_t bytes, hipStream_t s, void** out) { return acquire_work(g.work, bytes, s, out); }
 
-int release_work(Workspace& w, hipStream_t s) {
-  w.stream = s;
-  w.used = true;
+int release_work(hipStream_t s) {
+  g.work_stream = s;
+  g.work_used = true;
   return CF_OK;
 }
-int release_work(hipStream_t s) { return release_work(g.work, s); }
+
+// The transforms' workspace of stream s, or nullptr where there is none to have.
+// A call recorded into a graph would share it with whatever runs on s beside the
+// replays; hipStreamPerThread is a stream of its own in every thread under one
+// handle, which nothing orders.  (A stream destroyed and another one made under
+// its handle: the first has finished its work.)
+void* fft_workspace(hipStream_t s) {
+  if (s == hipStreamPerThread || capturing(s)) return nullptr;
+  for (const FftWork& w : g.fft_work)
+    if (w.stream == s) return w.d;
+  if (g.fft_work.size() >= kFftWorkStreams) return nullptr;
+  void* d = nullptr;
+  if (dev_malloc(&d, kFftWorkBytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  g.fft_work.push_back({s, d});
+  return d;
+}
 
 int ensure_events() {
   for (auto& e : g.ev)
@@ -2028,25 +2056,11 @@ extern "C" int cf_fft3d_device(unsigned n, const void* d_in, void* d_out, unsign
   CFCHK(size_res(n, &f));
   hipStream_t s = (hipStream_t)stream;
   const unsigned group = pass_group(n, how_many, kTransformSlack);
-  // 256^3 in two passes through the workspace (97 us against 133 forward, 143
+  // 256^3 in two passes through the stream's workspace (97 us against 133 forward, 143
   // inverse in one pass per axis), 512^3 by slabs (1073 against 1230 forward, 1157
-  // against 1245 inverse).  A call recorded into a graph would share the workspace
-  // with whatever runs beside its replays, and cannot allocate it: it keeps the axis
-  // passes, as does a call that finds no memory for it, and one on hipStreamPerThread,
-  // a stream of its own in every thread under one handle, which nothing orders.
-  void* work = nullptr;
+  // against 1245 inverse); without one, the axis passes
   const size_t need = fft_work_bytes(n, group);
-  if (need && s != hipStreamPerThread && !capturing(s) && acquire_work(g.fft_work, need, s, &work) != CF_OK) {
-    (void)hipGetLastError();
-    work = nullptr;
-  }
-  struct WorkRelease {
-    void* w;
-    hipStream_t s;
-    ~WorkRelease() {
-      if (w) release_work(g.fft_work, s);
-    }
-  } wr{work, s};
+  void* work = need && need <= kFftWorkBytes ? fft_workspace(s) : nullptr;
   for (unsigned b = 0; b < how_many; b += group) {
     const unsigned nb = std::min(group, how_many - b);
     const void* in = (const char*)d_in + b * cube_bytes(n);

@@ -49,11 +49,49 @@ static void fft_per_thread() {
     }
 }
 
+// Transforms on different streams have nothing to do with each other: no memory in
+// common, no order between them, no wait, whatever was queued or is being captured
+// on the others.
+static void fft_streams() {
+  for (unsigned n : {256u, 512u}) {
+    hipStream_t s[6];
+    for (auto& x : s) x = rec::new_stream();
+    forget();
+    for (auto x : s) {
+      Bufs b(n);
+      for (int k = 0; k < 2; ++k) CHECK(fft(n, b, x, k) == CF_OK);
+    }
+    CHECK(rec::races() == 0);
+    CHECK(rec::faults.empty() && rec::device_waits == 0);
+    for (auto& a : rec::launches)
+      for (auto& b : rec::launches) CHECK(a.stream == b.stream || !rec::ordered(a, b));
+  }
+}
+static void fft_beside_capture() {
+  for (unsigned n : {256u, 512u}) {
+    hipStream_t a = rec::new_stream(), b = rec::new_stream();
+    Bufs x(n), y(n);
+    fft(n, y, b);
+    fft(n, x, a);  // the last user of what transforms may share
+    forget();
+    rec::begin_capture(a);
+    CHECK(fft(n, x, a) == CF_OK);
+    CHECK(rec::captured_launches > 0 && rec::launches.empty());
+    const unsigned captured = rec::captured_launches;
+    CHECK(fft(n, y, b) == CF_OK);
+    rec::end_capture(a);
+    CHECK(rec::faults.empty());
+    CHECK(rec::captured_launches == captured && !rec::launches.empty());
+  }
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
     void (*run)();
-  } checks[] = {{"fft_per_thread", fft_per_thread}};
+  } checks[] = {{"fft_per_thread", fft_per_thread},
+                {"fft_streams", fft_streams},
+                {"fft_beside_capture", fft_beside_capture}};
   CHECK(fpga_initialize("gfx950", "recorded", false) == 0);
   bool found = false;
   for (auto& c : checks)

@@ -9,10 +9,10 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
-CHECKS = ["fft_per_thread"]
+CHECKS = ["fft_per_thread", "fft_streams", "fft_beside_capture"]
 
-pytestmark = pytest.mark.skipif(shutil.which("g++") is None or not os.path.exists(os.path.join(ROCM, "include", "hip")),
-                                reason="needs g++ and the HIP headers")
+needs_gxx = pytest.mark.skipif(shutil.which("g++") is None or not os.path.exists(os.path.join(ROCM, "include", "hip")),
+                               reason="needs g++ and the HIP headers")
 
 
 @pytest.fixture(scope="module")
@@ -26,7 +26,85 @@ def check(tmp_path_factory):
     return str(exe)
 
 
+@needs_gxx
 @pytest.mark.parametrize("name", CHECKS)
 def test_stream_order(check, name):
     r = subprocess.run([check, name], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.endswith("ok %s\n" % name), r.stdout
+
+
+def _transforms(n, k):
+    """k inputs and what one call on each gives, by whichever route"""
+    import torch
+    import convfpga_amd as C
+    x = torch.empty((k, n, n, n), dtype=torch.complex64, device="cuda")
+    C.api.fill_uniform(x, 2 * x.numel(), 73001 + n)
+    want = torch.stack([torch.fft.fftn(v.to(torch.complex128)) for v in x])
+    return x, torch.empty_like(x), want
+
+
+def _rel(a, b):
+    import torch
+    return max(float(torch.linalg.vector_norm(p.to(torch.complex128) - q) / torch.linalg.vector_norm(q))
+               for p, q in zip(a, b))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("per_thread", [True, False])
+def test_transforms_of_several_threads(gpu, per_thread):
+    """256^3 transforms of six threads, on hipStreamPerThread (handle 2) or on a
+    stream each (two more than there are workspaces), held to the FP32 bound of the
+    other transform tests."""
+    import threading
+
+    import torch
+    n, k, rounds = 256, 6, 8
+    print("case fft threads per_thread=%s" % per_thread, flush=True)
+    x, y, want = _transforms(n, k)
+    streams = [2 if per_thread else torch.cuda.Stream() for _ in range(k)]
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(i):
+        try:
+            for _ in range(rounds):
+                gpu.fft3d_device(n, x[i], y[i], stream=streams[i])
+            torch.cuda.synchronize()
+        except Exception as e:  # shown by the assertion below
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(k)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors and _rel(y, want) <= 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [256, 512])
+def test_transform_beside_a_capture(gpu, n):
+    """A stream that ran a transform is recorded into a graph while another stream
+    runs one: that one runs at once, and the graph is whole."""
+    import torch
+    print("case fft beside capture N=%d" % n, flush=True)
+    x, y, want = _transforms(n, 2)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    gpu.fft3d_device(n, x[1], y[1], stream=b)
+    gpu.fft3d_device(n, x[0], y[0], stream=a)
+    torch.cuda.synchronize()
+    y.fill_(float("nan"))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=a, capture_error_mode="relaxed"):
+        gpu.fft3d_device(n, x[0], y[0], stream=a)
+        gpu.fft3d_device(n, x[1], y[1], stream=b)
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(torch.view_as_real(y[0])).all()) and _rel(y[1:], want[1:]) <= 1e-5
+    for _ in range(3):
+        y.fill_(float("nan"))
+        graph.replay()
+        gpu.fft3d_device(n, x[1], y[1])
+        torch.cuda.synchronize()
+        assert _rel(y, want) <= 1e-5
