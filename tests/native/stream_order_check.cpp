@@ -85,13 +85,38 @@ static void fft_beside_capture() {
   }
 }
 
+// A stream's first transform, which makes its workspace, is as free to be called as
+// a later one: beside a capture, with no memory left, and with nothing waited for.
+static void fft_first_call() {
+  for (unsigned n : {256u, 512u}) {
+    Bufs x(n), y(n);
+    cf_spectrum_t kept = nullptr;
+    CHECK(cf_set_plan(n, CF_PLAN_AXIS5) == CF_OK);
+    CHECK(cf_spectrum_create(n, 1, x.in, 1, nullptr, &kept) == CF_OK);
+    cf_spectrum_destroy(kept);
+    hipStream_t a = rec::new_stream();
+    forget();
+    rec::begin_capture(a);
+    CHECK(fft(n, y, rec::new_stream()) == CF_OK);
+    rec::end_capture(a);
+    CHECK(rec::faults.empty() && rec::device_waits == 0 && rec::launches.size() > 0);
+    CHECK(cf_set_plan(7, CF_PLAN_AUTO) < 0);
+    const std::string text = cf_last_error();
+    rec::alloc_limit = 0;
+    CHECK(fft(n, y, rec::new_stream()) == CF_OK);
+    rec::alloc_limit = ~size_t(0);
+    CHECK(rec::device_waits == 0 && text == cf_last_error() && hipGetLastError() == hipSuccess);
+  }
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
     void (*run)();
   } checks[] = {{"fft_per_thread", fft_per_thread},
                 {"fft_streams", fft_streams},
-                {"fft_beside_capture", fft_beside_capture}};
+                {"fft_beside_capture", fft_beside_capture},
+                {"fft_first_call", fft_first_call}};
   CHECK(fpga_initialize("gfx950", "recorded", false) == 0);
   bool found = false;
   for (auto& c : checks)

@@ -9,7 +9,7 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
-CHECKS = ["fft_per_thread", "fft_streams", "fft_beside_capture"]
+CHECKS = ["fft_per_thread", "fft_streams", "fft_beside_capture", "fft_first_call"]
 
 needs_gxx = pytest.mark.skipif(shutil.which("g++") is None or not os.path.exists(os.path.join(ROCM, "include", "hip")),
                                reason="needs g++ and the HIP headers")
@@ -33,6 +33,14 @@ def test_stream_order(check, name):
     assert r.returncode == 0 and r.stdout.endswith("ok %s\n" % name), r.stdout
 
 
+@pytest.fixture
+def fresh(gpu):
+    """the library as a program that has just started finds it: no stream has a workspace"""
+    gpu.fpga_final()
+    assert gpu.fpga_initialize("gfx950", gpu.CODE_OBJECT, True) == 0
+    return gpu
+
+
 def _transforms(n, k):
     """k inputs and what one call on each gives, by whichever route"""
     import torch
@@ -51,7 +59,7 @@ def _rel(a, b):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("per_thread", [True, False])
-def test_transforms_of_several_threads(gpu, per_thread):
+def test_transforms_of_several_threads(fresh, per_thread):
     """256^3 transforms of six threads, on hipStreamPerThread (handle 2) or on a
     stream each (two more than there are workspaces), held to the FP32 bound of the
     other transform tests."""
@@ -68,7 +76,7 @@ def test_transforms_of_several_threads(gpu, per_thread):
     def work(i):
         try:
             for _ in range(rounds):
-                gpu.fft3d_device(n, x[i], y[i], stream=streams[i])
+                fresh.fft3d_device(n, x[i], y[i], stream=streams[i])
             torch.cuda.synchronize()
         except Exception as e:  # shown by the assertion below
             errors.append(e)
@@ -83,7 +91,7 @@ def test_transforms_of_several_threads(gpu, per_thread):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [256, 512])
-def test_transform_beside_a_capture(gpu, n):
+def test_transform_beside_a_capture(fresh, n):
     """A stream that ran a transform is recorded into a graph while another stream
     runs one: that one runs at once, and the graph is whole."""
     import torch
@@ -91,20 +99,47 @@ def test_transform_beside_a_capture(gpu, n):
     x, y, want = _transforms(n, 2)
     a, b = torch.cuda.Stream(), torch.cuda.Stream()
     torch.cuda.synchronize()
-    gpu.fft3d_device(n, x[1], y[1], stream=b)
-    gpu.fft3d_device(n, x[0], y[0], stream=a)
+    fresh.fft3d_device(n, x[1], y[1], stream=b)
+    fresh.fft3d_device(n, x[0], y[0], stream=a)
     torch.cuda.synchronize()
     y.fill_(float("nan"))
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=a, capture_error_mode="relaxed"):
-        gpu.fft3d_device(n, x[0], y[0], stream=a)
-        gpu.fft3d_device(n, x[1], y[1], stream=b)
+        fresh.fft3d_device(n, x[0], y[0], stream=a)
+        fresh.fft3d_device(n, x[1], y[1], stream=b)
     torch.cuda.synchronize()
     assert bool(torch.isnan(y[0]).all()) and _rel(y[1:], want[1:]) <= 1e-5
     for _ in range(3):
         y.fill_(float("nan"))
         graph.replay()
-        gpu.fft3d_device(n, x[1], y[1])
+        fresh.fft3d_device(n, x[1], y[1])
+        torch.cuda.synchronize()
+        assert _rel(y, want) <= 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["global", "thread_local", "relaxed"])
+def test_first_transform_of_a_stream_beside_a_capture(fresh, mode):
+    """A stream's first 256^3 transform, which allocates its workspace, while
+    another stream is recorded into a graph."""
+    import torch
+    n = 256
+    print("case first fft beside capture mode=%s" % mode, flush=True)
+    x, y, want = _transforms(n, 2)
+    fresh.fft3d_device(n, x[0], y[0])
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()  # (as torch.cuda.graph does)
+    free = torch.cuda.mem_get_info()[0]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=a, capture_error_mode=mode):
+        fresh.fft3d_device(n, x[0], y[0], stream=a)
+        fresh.fft3d_device(n, x[1], y[1], stream=b)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] >= 256 << 20  # the workspace
+    for _ in range(3):
+        y[0].fill_(float("nan"))
+        graph.replay()
         torch.cuda.synchronize()
         assert _rel(y, want) <= 1e-5
