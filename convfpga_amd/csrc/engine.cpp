@@ -16,6 +16,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cctype>
 #include <chrono>
 #include <cmath>
@@ -194,6 +195,8 @@ struct Engine {
   hipStream_t work_stream = nullptr;
   bool work_used = false;
   hipEvent_t work_ev = nullptr;
+  unsigned long long work_thread = 0;  // of the last user, if its stream is hipStreamPerThread,
+  bool work_recorded = false;          // and whether work_ev was recorded after its use
   std::vector<FftWork> fft_work;
   std::vector<SpecMem> spec_pool;
   std::string arch;
@@ -958,6 +961,13 @@ double host_ms(std::chrono::steady_clock::time_point a, std::chrono::steady_cloc
   return std::chrono::duration<double, std::milli>(b - a).count();
 }
 
+// The calling thread's number (unlike its id, never that of a thread that has ended).
+unsigned long long thread_number() {
+  static std::atomic<unsigned long long> last{0};
+  thread_local const unsigned long long mine = ++last;
+  return mine;
+}
+
 // Workspace of `bytes` for a call on stream s.  Calls on different streams are
 // ordered through work_ev so that they never overlap on the shared workspace.
 int acquire_work(size_t bytes, hipStream_t s, void** out) {
@@ -974,14 +984,18 @@ int acquire_work(size_t bytes, hipStream_t s, void** out) {
     if (e != hipSuccess) return fail(CF_ERR_NOMEM, "hipMalloc(%zu) for the workspace: %s", bytes, hipGetErrorString(e));
     g.d_work_bytes = bytes;
   }
-  if (g.work_used && g.work_stream != s) {
+  // (hipStreamPerThread is another stream in every thread, which only its own thread
+  // can record an event on: there release_work has recorded it)
+  const bool per_thread = g.work_stream == hipStreamPerThread;
+  const bool same = g.work_stream == s && (!per_thread || g.work_thread == thread_number());
+  if (g.work_used && !same) {
     // Everything submitted so far to the previous user's stream includes its
     // use of the workspace, so an event recorded there now orders s after it.
     // (Recording lazily, only on a change of stream, keeps event packets --
     // each a gap of several microseconds on the GPU -- out of the
     // single-stream sequence.)  A stream destroyed meanwhile has finished its
     // work; should the record fail, wait for the whole device instead.
-    if (hipEventRecord(g.work_ev, g.work_stream) == hipSuccess) {
+    if (per_thread ? g.work_recorded : hipEventRecord(g.work_ev, g.work_stream) == hipSuccess) {
       HIPCHK(hipStreamWaitEvent(s, g.work_ev, 0));
     } else {
       (void)hipGetLastError();
@@ -995,6 +1009,10 @@ int acquire_work(size_t bytes, hipStream_t s, void** out) {
 int release_work(hipStream_t s) {
   g.work_stream = s;
   g.work_used = true;
+  if (s == hipStreamPerThread) {
+    g.work_thread = thread_number();
+    g.work_recorded = !capturing(s) && hipEventRecord(g.work_ev, s) == hipSuccess;
+  }
   return CF_OK;
 }
 

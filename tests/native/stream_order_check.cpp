@@ -109,6 +109,31 @@ static void fft_first_call() {
   }
 }
 
+// Convolutions through the common workspace (a four-step plan) are ordered, whoever
+// calls: threads on their hipStreamPerThread, other streams before and after them.
+static void conv_per_thread() {
+  CHECK(cf_set_plan(256, CF_PLAN_SPLIT3_G24) == CF_OK);
+  Bufs f(256), x(256), y(256), z(256);
+  cf_spectrum_t h = nullptr;
+  CHECK(cf_spectrum_create(256, 1, f.in, 1, nullptr, &h) == CF_OK);
+  hipStream_t s = rec::new_stream();
+  forget();
+  auto conv = [&](const Bufs& b, hipStream_t st) {
+    CHECK(cf_conv3d_device(h, b.in, b.out, 1, CF_SCALE_INV_N3, CF_PREC_FP32, st) == CF_OK);
+  };
+  conv(z, s);
+  for (int k = 0; k < 2; ++k) {
+    std::thread([&] { conv(x, hipStreamPerThread), conv(x, hipStreamPerThread); }).join();
+    std::thread([&] { conv(y, hipStreamPerThread); }).join();
+    if (k == 0) conv(z, s);
+  }
+  conv(z, nullptr);
+  CHECK(rec::launches.size() == 3 * 9);
+  CHECK(rec::races() == 0);
+  CHECK(rec::faults.empty() && rec::device_waits == 0);
+  cf_spectrum_destroy(h);
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
@@ -116,7 +141,8 @@ int main(int argc, char** argv) {
   } checks[] = {{"fft_per_thread", fft_per_thread},
                 {"fft_streams", fft_streams},
                 {"fft_beside_capture", fft_beside_capture},
-                {"fft_first_call", fft_first_call}};
+                {"fft_first_call", fft_first_call},
+                {"conv_per_thread", conv_per_thread}};
   CHECK(fpga_initialize("gfx950", "recorded", false) == 0);
   bool found = false;
   for (auto& c : checks)

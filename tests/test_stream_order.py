@@ -9,7 +9,7 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
-CHECKS = ["fft_per_thread", "fft_streams", "fft_beside_capture", "fft_first_call"]
+CHECKS = ["fft_per_thread", "fft_streams", "fft_beside_capture", "fft_first_call", "conv_per_thread"]
 
 needs_gxx = pytest.mark.skipif(shutil.which("g++") is None or not os.path.exists(os.path.join(ROCM, "include", "hip")),
                                reason="needs g++ and the HIP headers")
@@ -143,3 +143,45 @@ def test_first_transform_of_a_stream_beside_a_capture(fresh, mode):
         graph.replay()
         torch.cuda.synchronize()
         assert _rel(y, want) <= 1e-5
+
+
+@pytest.mark.gpu
+def test_convolutions_of_several_threads(fresh):
+    """256^3 convolutions through the common workspace from four threads on their
+    hipStreamPerThread (handle 2), with others on a stream between them: the bits of
+    calls one after the other."""
+    import threading
+
+    import torch
+    api, n, k, rounds = fresh.api, 256, 5, 8
+    print("case conv threads", flush=True)
+    x = torch.empty((k, n, n, n), dtype=torch.complex64, device="cuda")
+    api.fill_uniform(x, 2 * x.numel(), 74001)
+    y, want = torch.empty_like(x), torch.empty_like(x)
+    api.set_plan(n, api.CF_PLAN_SPLIT3_G24)
+    try:
+        spec = fresh.Spectrum(n, x[0])
+    finally:
+        api.set_plan(n, api.CF_PLAN_AUTO)
+    for i in range(k):
+        fresh.conv3d_device(spec, x[i], want[i])
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(i):
+        try:
+            for _ in range(rounds):
+                fresh.conv3d_device(spec, x[i], y[i], stream=2 if i else stream)
+            torch.cuda.synchronize()
+        except Exception as e:  # shown by the assertion below
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(k)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    spec.close()
+    assert not errors
+    assert torch.equal(torch.view_as_real(y).view(torch.int32), torch.view_as_real(want).view(torch.int32))
