@@ -1658,16 +1658,16 @@ struct cf_spectrum_s {
   std::shared_ptr<SpecMem> mem;  // that memory (a view's: its parent's)
 };
 
-// Memory for a spectrum that stream s will write: a kept block of the size, if
-// there is one and (unless only s can still be reading it) after waiting for
-// the device; otherwise new.
+// Memory for a spectrum that stream s will write: a kept block of the size that
+// nothing but s can still be reading, if there is one, otherwise new.  (Waiting for
+// the readers of another block could hold the caller for work that has nothing to do
+// with this spectrum, and would end any capture.)
 static int spec_mem_get(size_t bytes, hipStream_t s, SpecMem* m) {
   for (size_t i = 0; i < g.spec_pool.size(); ++i) {
-    if (g.spec_pool[i].bytes != bytes) continue;
-    const SpecMem old = g.spec_pool[i];
-    if (old.many || (old.used && (old.stream != s || s == hipStreamPerThread))) HIPCHK(hipDeviceSynchronize());
-    g.spec_pool.erase(g.spec_pool.begin() + i);
+    const SpecMem& old = g.spec_pool[i];
+    if (old.bytes != bytes || (old.used && old.stream != s)) continue;
     m->d = old.d;
+    g.spec_pool.erase(g.spec_pool.begin() + i);
     m->bytes = bytes;
     return CF_OK;
   }
@@ -1677,8 +1677,10 @@ static int spec_mem_get(size_t bytes, hipStream_t s, SpecMem* m) {
   return CF_OK;
 }
 
+// Keeps a destroyed spectrum's memory, unless more than one stream, or others, may
+// be reading it: that is freed, which waits for them.
 static void spec_mem_put(const SpecMem& m) {
-  if (!g.ready || m.bytes > kSpecPoolBytes) {
+  if (!g.ready || m.many || m.bytes > kSpecPoolBytes) {
     (void)hipFree(m.d);
     return;
   }

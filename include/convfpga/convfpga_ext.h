@@ -108,9 +108,12 @@ int cf_autotune(unsigned N, float *ms);
  * The reference recomputes the filter transform in every call
  * (host/src/convfpga.c:87-172); a spectrum handle computes it once.
  * `count` filters of edge N, contiguous, on the host or the device.
- * cf_spectrum_destroy does not wait for convolutions still queued with the
- * spectrum; its memory is kept for later spectra of the size (four at most, 1
- * GiB in all) until an allocation of this library needs it or fpga_final(). */
+ * cf_spectrum_destroy frees a spectrum that several streams, a batch or a
+ * recorded call used, or whose address was taken, and then waits for the device.
+ * Otherwise it does not wait for convolutions still queued with the spectrum:
+ * its memory is kept for later spectra of the size made on the same stream (four
+ * at most, 1 GiB in all) until an allocation of this library needs it or
+ * fpga_final(). */
 typedef struct cf_spectrum_s *cf_spectrum_t;
 int cf_spectrum_create(unsigned N, unsigned count, const void *filters, int on_device, void *stream,
                        cf_spectrum_t *out);

@@ -180,7 +180,11 @@ REC hipMemcpy(void*, const void*, size_t, hipMemcpyKind) { return rec::wait_all(
 REC hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
 REC hipMemset(void*, int, size_t) { return rec::wait_all(), hipSuccess; }
 REC hipDeviceSynchronize() {
-  if (rec::forbidden("hipDeviceSynchronize")) return rec::ret(hipErrorStreamCaptureUnsupported);
+  for (rec::Stream* s : rec::streams)  // (in every mode)
+    if (s->capturing) {
+      rec::faults.push_back("hipDeviceSynchronize during a capture");
+      return rec::ret(hipErrorStreamCaptureUnsupported);
+    }
   return rec::wait_all(), hipSuccess;
 }
 REC hipStreamCreate(hipStream_t* s) { return *s = rec::new_stream(), hipSuccess; }

@@ -134,6 +134,57 @@ static void conv_per_thread() {
   cf_spectrum_destroy(h);
 }
 
+// A destroyed spectrum's memory is written again only after the convolutions queued
+// with it: at once on the one stream that used it, which orders them; on no other.
+// What several streams, or others, may be reading is freed, which waits for them.
+// Making a spectrum waits for no stream but its own.
+static void spectrum_reuse() {
+  CHECK(cf_set_plan(128, CF_PLAN_AXIS5) == CF_OK);
+  Bufs f(128), x(128), y(128);
+  hipStream_t a = rec::new_stream(), b = rec::new_stream(), capture = rec::new_stream();
+  auto make = [&](hipStream_t s) {
+    cf_spectrum_t h = nullptr;
+    CHECK(cf_spectrum_create(128, 1, f.in, 1, s, &h) == CF_OK);
+    return h;
+  };
+  auto conv = [&](cf_spectrum_t h, const Bufs& u, hipStream_t s) {
+    CHECK(cf_conv3d_device(h, u.in, u.out, 1, CF_SCALE_INV_N3, CF_PREC_FP32, s) == CF_OK);
+  };
+  enum { ONE, TWO_STREAMS, PER_THREAD, ADDRESS, CAPTURED, VIEW };
+  make(a);  // (the edge is set up)
+  for (int use : {ONE, TWO_STREAMS, PER_THREAD, ADDRESS, CAPTURED, VIEW})
+    for (hipStream_t next : {a, b, (hipStream_t)hipStreamPerThread}) {
+      cf_spectrum_t h = make(a), v = h;
+      forget();
+      const size_t blocks = rec::allocs.size();
+      if (use == VIEW) CHECK(cf_spectrum_view(h, 0, &v) == CF_OK);
+      conv(v, x, a);
+      if (use == TWO_STREAMS) conv(h, y, b);
+      if (use == PER_THREAD) conv(h, y, hipStreamPerThread);
+      if (use == ADDRESS) CHECK(cf_spectrum_data(h) != nullptr);
+      if (use == CAPTURED) {
+        rec::begin_capture(capture, hipStreamCaptureModeRelaxed);
+        conv(h, y, capture);
+        rec::end_capture(capture);
+      }
+      if (v != h) cf_spectrum_destroy(v);
+      const bool sole = use == ONE || use == VIEW;
+      cf_spectrum_destroy(h);
+      CHECK(rec::device_waits == (sole ? 0 : 1));
+      rec::begin_capture(capture, hipStreamCaptureModeRelaxed);  // which a wait for the device would end
+      rec::mode = hipStreamCaptureModeRelaxed;
+      h = make(next);
+      rec::mode = hipStreamCaptureModeGlobal;
+      rec::end_capture(capture);
+      CHECK(rec::device_waits == (sole ? 0 : 1));
+      if (use == ONE && next == a) CHECK(rec::allocs.size() == blocks);
+      conv(h, y, next);
+      CHECK(rec::races() == 0 && rec::faults.empty());
+      CHECK(cf_spectrum_data(h) != nullptr);  // (freed, not kept)
+      cf_spectrum_destroy(h);
+    }
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
@@ -142,7 +193,8 @@ int main(int argc, char** argv) {
                 {"fft_streams", fft_streams},
                 {"fft_beside_capture", fft_beside_capture},
                 {"fft_first_call", fft_first_call},
-                {"conv_per_thread", conv_per_thread}};
+                {"conv_per_thread", conv_per_thread},
+                {"spectrum_reuse", spectrum_reuse}};
   CHECK(fpga_initialize("gfx950", "recorded", false) == 0);
   bool found = false;
   for (auto& c : checks)

@@ -53,3 +53,46 @@ def test_kept_memory_is_bounded(gpu):
     for s in specs:
         s.close()
     assert free0 - torch.cuda.mem_get_info()[0] <= 1 << 30
+
+
+@pytest.mark.parametrize("n,count", [(64, 37), (128, 5), (256, 3)])
+@pytest.mark.parametrize("other_stream", [False, True])
+def test_old_spectrum_is_read_while_the_next_is_made(gpu, n, count, other_stream):
+    """The only kept block of a size is that of a spectrum whose convolutions are
+    still queued when the next spectrum of the size is made, on the same or on
+    another stream: the last of them, which runs after that, has the old values.
+    (Five passes without a workspace, which would order the streams.)"""
+    import torch
+    api = gpu.api
+    print("case spectrum read N=%d count=%d other_stream=%s" % (n, count, other_stream), flush=True)
+    gpu.fpga_final()  # nothing is kept: closing a fifth spectrum would free the oldest one, and wait
+    assert gpu.fpga_initialize("gfx950", gpu.CODE_OBJECT, True) == 0
+    api.set_plan(n, api.CF_PLAN_AXIS5)
+    try:
+        filt = torch.empty((2, count, n ** 3), dtype=torch.complex64, device="cuda")
+        sig = torch.empty((count, n ** 3), dtype=torch.complex64, device="cuda")
+        api.fill_uniform(filt, 2 * filt.numel(), 67001 + n)
+        api.fill_uniform(sig, 2 * sig.numel(), 67002 + n)
+        want, out = torch.empty_like(filt), torch.empty_like(filt)
+        for k in range(2):
+            spec = gpu.Spectrum(n, filt[k], count)
+            gpu.conv3d_device(spec, sig, want[k], count)
+            spec.data_ptr()  # the address is taken: freed, not kept
+            spec.close()
+        a = torch.cuda.Stream()
+        b = torch.cuda.Stream() if other_stream else a
+        torch.cuda.synchronize()
+        old = gpu.Spectrum(n, filt[0], count, stream=a)
+        for _ in range(200):
+            gpu.conv3d_device(old, sig, out[0], count, stream=a)
+        queued = torch.cuda.Event()
+        queued.record(a)
+        old.close()
+        new = gpu.Spectrum(n, filt[1], count, stream=b)
+        assert not other_stream or not queued.query()
+        gpu.conv3d_device(new, sig, out[1], count, stream=b)
+        torch.cuda.synchronize()
+        new.close()
+    finally:
+        api.set_plan(n, api.CF_PLAN_AUTO)
+    assert torch.equal(_bits(out), _bits(want))
