@@ -118,14 +118,16 @@ bool plan_ok(unsigned n, int plan) {
 // stream has its own, so that transforms on different streams stay independent
 // (no order between them, and no call on a stream that may be recording a graph)
 // and meet neither the convolutions' workspace nor a graph that holds the address
-// of that one.  At most kFftWorkStreams of them, for the streams that come first;
-// transforms on others run one pass per axis, as without a workspace.
+// of that one.  Nor is it taken from one stream for another: whether a stream has
+// finished with it could only be asked of the stream, which may be destroyed by
+// then.  kFftWorkTotal in all (16 streams at 256^3, 8 at 512^3), for the streams that
+// come first; transforms on others run one pass per axis, as without a workspace.
 struct FftWork {
   hipStream_t stream;
+  size_t bytes;
   void* d;
 };
-constexpr size_t kFftWorkStreams = 4;
-constexpr size_t kFftWorkBytes = std::max<size_t>(cfgeo::slab_bytes, size_t(8) << 24);  // a 512^3 slab, a 256^3 cube
+constexpr size_t kFftWorkTotal = size_t(2) << 30;
 
 // true if calls on s are being recorded into a graph (or that cannot be told)
 bool capturing(hipStream_t s) {
@@ -1016,30 +1018,33 @@ int release_work(hipStream_t s) {
   return CF_OK;
 }
 
-// The transforms' workspace of stream s, or nullptr where there is none to have.
+// The transforms' workspace of `bytes` for stream s, or nullptr where there is none to have.
 // A call recorded into a graph would share it with whatever runs on s beside the
 // replays; hipStreamPerThread is a stream of its own in every thread under one
 // handle, which nothing orders.  (A stream made under a destroyed one's
 // handle finds the workspace idle: hipStreamDestroy waits, 43 ms with 300
 // convolutions queued.)
-void* fft_workspace(hipStream_t s) {
+void* fft_workspace(size_t bytes, hipStream_t s) {
   if (s == hipStreamPerThread || capturing(s)) return nullptr;
-  for (const FftWork& w : g.fft_work)
-    if (w.stream == s) return w.d;
-  if (g.fft_work.size() >= kFftWorkStreams) return nullptr;
+  size_t total = bytes;
+  for (const FftWork& w : g.fft_work) {
+    if (w.stream == s && w.bytes >= bytes) return w.d;
+    total += w.bytes;
+  }
+  if (total > kFftWorkTotal) return nullptr;
   // relaxed: a transform only launches kernels on s, which another stream's capture
   // does not forbid, as it would this allocation; hipMalloc alone, since giving kept
   // spectra back would wait for the device
   void* d = nullptr;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
-  const hipError_t e = hipMalloc(&d, kFftWorkBytes);
+  const hipError_t e = hipMalloc(&d, bytes);
   (void)hipThreadExchangeStreamCaptureMode(&mode);
   if (e != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
-  g.fft_work.push_back({s, d});
+  g.fft_work.push_back({s, bytes, d});
   return d;
 }
 
@@ -2088,7 +2093,7 @@ extern "C" int cf_fft3d_device(unsigned n, const void* d_in, void* d_out, unsign
   // inverse in one pass per axis), 512^3 by slabs (1073 against 1230 forward, 1157
   // against 1245 inverse); without one, the axis passes
   const size_t need = fft_work_bytes(n, group);
-  void* work = need && need <= kFftWorkBytes ? fft_workspace(s) : nullptr;
+  void* work = need ? fft_workspace(need, s) : nullptr;
   for (unsigned b = 0; b < how_many; b += group) {
     const unsigned nb = std::min(group, how_many - b);
     const void* in = (const char*)d_in + b * cube_bytes(n);

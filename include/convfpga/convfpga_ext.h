@@ -257,10 +257,10 @@ int cf_batch_create_stall_test(const cf_instance_t *inst, unsigned count, int sc
 /* ---- plain 3D transforms (device) ------------------------------------------ */
 /* forward (inverse = 0) or unnormalised inverse (inverse = 1) 3D FFT.  Calls on
  * different streams are independent of each other.  N = 256 and 512 go through
- * a workspace of 256 MiB that belongs to the stream, made by its first such call
- * and kept until fpga_final(), for the first four streams; calls on further
- * streams, on hipStreamPerThread, or recorded into a graph run one pass per axis
- * without it (at N = 256 the two routes round differently). */
+ * a workspace (128 and 256 MiB) that belongs to the stream, made by its first
+ * such call and kept until fpga_final(), 2 GiB in all; calls on further streams,
+ * on hipStreamPerThread, or recorded into a graph run one pass per axis without
+ * it (at N = 256 the two routes round differently). */
 int cf_fft3d_device(unsigned N, const void *d_in, void *d_out, unsigned how_many, int inverse, void *stream);
 
 /* ---- FP64 error norm on the device -----------------------------------------

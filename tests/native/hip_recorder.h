@@ -52,7 +52,7 @@ inline std::vector<Stream*> streams;
 inline std::map<std::thread::id, Stream*> per_thread;
 inline Clock host;
 inline std::map<const char*, size_t> allocs;
-inline size_t alloc_limit = ~size_t(0);
+inline size_t held = 0, alloc_limit = ~size_t(0);  // bytes of hipMalloc, and the most of them
 inline std::vector<Launch> launches;
 inline unsigned captured_launches = 0, device_waits = 0;
 inline std::vector<std::string> faults;
@@ -161,16 +161,18 @@ extern "C" const char* hipGetErrorString(hipError_t) { return "recorded error"; 
 REC hipMalloc(void** p, size_t bytes) {
   *p = nullptr;
   if (rec::forbidden("hipMalloc")) return rec::ret(hipErrorStreamCaptureUnsupported);
-  size_t used = 0;
-  for (auto& a : rec::allocs) used += a.second;
-  if (bytes > rec::alloc_limit - std::min(used, rec::alloc_limit)) return rec::ret(hipErrorOutOfMemory);
+  if (rec::held + bytes > rec::alloc_limit) return rec::ret(hipErrorOutOfMemory);
+  rec::held += bytes;
   return *p = rec::alloc(bytes), hipSuccess;
 }
 REC hipFree(void* p) {
   if (!p) return hipSuccess;
   if (rec::forbidden("hipFree")) return rec::ret(hipErrorStreamCaptureUnsupported);
   rec::wait_all();
-  if (!rec::allocs.erase((char*)p)) rec::faults.push_back("hipFree of what is not allocated");
+  auto it = rec::allocs.find((char*)p);
+  if (it == rec::allocs.end()) return rec::faults.push_back("hipFree of what is not allocated"), hipSuccess;
+  rec::held -= it->second;
+  rec::allocs.erase(it);
   return hipSuccess;
 }
 REC hipHostMalloc(void** p, size_t bytes, unsigned) { return *p = malloc(bytes), hipSuccess; }

@@ -53,19 +53,25 @@ static void fft_per_thread() {
 // common, no order between them, no wait, whatever was queued or is being captured
 // on the others.
 static void fft_streams() {
-  for (unsigned n : {256u, 512u}) {
-    hipStream_t s[6];
-    for (auto& x : s) x = rec::new_stream();
+  hipStream_t s[20];
+  for (auto& x : s) x = rec::new_stream();
+  const size_t held = rec::held;
+  for (unsigned n : {256u, 512u, 256u}) {
     forget();
     for (auto x : s) {
       Bufs b(n);
       for (int k = 0; k < 2; ++k) CHECK(fft(n, b, x, k) == CF_OK);
     }
+    std::set<int> axis;  // the streams that have no workspace
+    for (auto& l : rec::launches)
+      if (l.name.rfind("cf_coly_inv_", 0) == 0 && l.name.find("slab") == std::string::npos) axis.insert(l.stream);
+    CHECK(axis.size() == (n == 256 ? 4 : 20));  // (16 at 256^3 leave nothing for 512^3)
     CHECK(rec::races() == 0);
     CHECK(rec::faults.empty() && rec::device_waits == 0);
     for (auto& a : rec::launches)
       for (auto& b : rec::launches) CHECK(a.stream == b.stream || !rec::ordered(a, b));
   }
+  CHECK(rec::held - held < (size_t(2) << 30) + (1 << 20));  // (and twiddles)
 }
 static void fft_beside_capture() {
   for (unsigned n : {256u, 512u}) {
