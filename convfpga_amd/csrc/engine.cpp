@@ -803,20 +803,34 @@ unsigned pass_group(unsigned n, unsigned count, unsigned slack) {
   return count / groups + (count % groups != 0);
 }
 
+// f(first cube, cubes) for every group of `count` cubes, from the last one if the
+// output lies above its signal in the same memory: a plan that takes a group's
+// signals into the workspace then reads every cube before its memory is written, as
+// with all cubes in one group.
+template <class F>
+int for_groups(unsigned n, unsigned count, unsigned group, const void* sig, const void* out, F f) {
+  const char *a = (const char*)sig, *b = (const char*)out;
+  const bool down = a < b && b < a + cube_bytes(n) * count;
+  const unsigned groups = count / group + (count % group != 0);
+  for (unsigned k = 0; k < groups; ++k) {
+    const unsigned first = (down ? groups - 1 - k : k) * group;
+    CFCHK(f(first, std::min(group, count - first)));
+  }
+  return CF_OK;
+}
+
 // The convolution passes over how_many cubes, group by group.  work holds the
 // intermediates of one group (work_bytes of pass_group(...) cubes).
 int run_conv(const SizeFns& f, int plan, unsigned n, unsigned how_many, const void* sig, void* out, void* work,
              const void* H, long long hstride, float scale, int precision, hipStream_t s) {
   const unsigned group = pass_group(n, how_many, conv_slack(plan, hstride != 0));
   const size_t V = cube_bytes(n);
-  for (unsigned b = 0; b < how_many; b += group) {
-    const unsigned nb = std::min(group, how_many - b);
+  return for_groups(n, how_many, group, sig, out, [&](unsigned b, unsigned nb) {
     PassList p;
     conv_passes(f, plan, n, nb, (const char*)sig + b * V, (char*)out + b * V, work,
                 (const char*)H + (size_t)b * hstride * 8, hstride, scale, p, precision);
-    CFCHK(run_passes(p, n, nb, s, f.tw, nullptr));
-  }
-  return CF_OK;
+    return run_passes(p, n, nb, s, f.tw, nullptr);
+  });
 }
 
 // One batch of a paired launch: cubes of edge n through the plane plan.
@@ -1866,8 +1880,8 @@ static int conv_device_impl(cf_spectrum_t h, const void* d_sig, void* d_out, uns
     memset(times, 0, sizeof *times);
   }
   const size_t V = cube_bytes(n);
-  for (unsigned b = 0; b < how_many; b += group) {
-    const unsigned nb = std::min(group, how_many - b);
+  bool named = false;
+  CFCHK(for_groups(n, how_many, group, d_sig, d_out, [&](unsigned b, unsigned nb) -> int {
     PassList p;
     conv_passes(*f, h->plan, n, nb, (const char*)d_sig + b * V, (char*)d_out + b * V, work,
                 (const char*)h->d + (size_t)b * hstride * 8, hstride, scale, p, precision);
@@ -1892,7 +1906,8 @@ static int conv_device_impl(cf_spectrum_t h, const void* d_sig, void* d_out, uns
         times->bytes[k] += p[i].bytes;
       }
     } else if (first) {
-      if (b == 0) {
+      if (!named) {
+        named = true;
         g.prof_npass = p.slots();
         g.prof_names.assign(p.slots(), "");
         g.prof_bytes.assign(p.slots(), 0.0);
@@ -1904,7 +1919,8 @@ static int conv_device_impl(cf_spectrum_t h, const void* d_sig, void* d_out, uns
         g.prof_bytes[x.slot] += x.bytes;
       }
     }
-  }
+    return CF_OK;
+  }));
   if (profiled) ++g.prof_calls;
   return CF_OK;
 }

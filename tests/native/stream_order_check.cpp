@@ -191,6 +191,55 @@ static void spectrum_reuse() {
     }
 }
 
+// A batch whose output overlaps its signal at another place: a plan that takes the
+// signal into the workspace reads every cube before it is overwritten.
+static void conv_overlap() {
+  const struct {
+    unsigned n, plan, count;
+    int precision;
+  } cases[] = {{128, CF_PLAN_SPLIT3_G24, 20, CF_PREC_FP32},
+               {256, CF_PLAN_SPLIT3_G24, 4, CF_PREC_FP32},
+               {256, CF_PLAN_SPLIT3_G24M2, 4, CF_PREC_SPLIT_FP16}};
+  for (auto& c : cases)
+    for (unsigned own : {0u, 1u})
+      for (bool timed : {false, true})
+        for (double shift : {1.0, -1.0, 2.5, -2.5, (double)c.count}) {
+          const size_t V = cube(c.n);
+          char* const buf = rec::alloc(V * 3 * c.count);
+          char* const sig = buf + V * c.count;
+          char* const out = sig + (long long)(shift * V);
+          cf_spectrum_t h = nullptr, one = nullptr;
+          CHECK(cf_set_plan(c.n, c.plan) == CF_OK);
+          CHECK(cf_spectrum_create(c.n, own ? c.count : 1, rec::alloc(V * c.count), 1, nullptr, &h) == CF_OK);
+          CHECK(cf_spectrum_create(c.n, 1, rec::alloc(V), 1, nullptr, &one) == CF_OK);
+          Bufs single(c.n);
+          forget();
+          CHECK(cf_conv3d_device(one, single.in, single.out, 1, CF_SCALE_INV_N3, c.precision, nullptr) == CF_OK);
+          std::map<std::string, int> tiles;
+          for (auto& l : rec::launches) tiles[l.name] = l.ntotal;
+          forget();
+          cf_pass_times_t t;
+          CHECK((timed ? cf_conv3d_device_timed(h, sig, out, c.count, CF_SCALE_INV_N3, c.precision, nullptr, &t)
+                       : cf_conv3d_device(h, sig, out, c.count, CF_SCALE_INV_N3, c.precision, nullptr)) == CF_OK);
+          unsigned read = 0, written = 0;
+          for (size_t j = 0; j < rec::launches.size(); ++j) {
+            const rec::Launch& l = rec::launches[j];
+            const unsigned nb = l.ntotal / tiles[l.name];
+            if (rec::base(l.out) == buf) written += nb;
+            if (rec::base(l.in) != buf) continue;
+            read += nb;
+            for (size_t i = 0; i <= j; ++i) {
+              const rec::Launch& w = rec::launches[i];
+              if (rec::base(w.out) == buf)
+                CHECK(w.out >= l.in + nb * V || l.in >= w.out + w.ntotal / tiles[w.name] * V);
+            }
+          }
+          CHECK(read == c.count && written == c.count);
+          cf_spectrum_destroy(h);
+          cf_spectrum_destroy(one);
+        }
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
@@ -200,7 +249,8 @@ int main(int argc, char** argv) {
                 {"fft_beside_capture", fft_beside_capture},
                 {"fft_first_call", fft_first_call},
                 {"conv_per_thread", conv_per_thread},
-                {"spectrum_reuse", spectrum_reuse}};
+                {"spectrum_reuse", spectrum_reuse},
+                {"conv_overlap", conv_overlap}};
   CHECK(fpga_initialize("gfx950", "recorded", false) == 0);
   bool found = false;
   for (auto& c : checks)

@@ -240,3 +240,33 @@ def test_batches_of_the_wide_plan(gpu, n, in_place):
         assert _same(out, ref)
     for h in [spec, shared] + singles:
         h.close()
+
+
+@pytest.mark.parametrize("n,count", [(128, 20), (256, 3)])
+@pytest.mark.parametrize("shift", [1, -1, 2.5])
+@pytest.mark.parametrize("own", [False, True])
+def test_groups_with_overlapping_output(gpu, n, count, shift, own):
+    """The output of a batch lies `shift` cubes from its signal in the same memory: a
+    plan that takes the signals into the workspace gives the bits of a call with
+    buffers of their own, as if all cubes were one group."""
+    import torch
+    api = gpu.api
+    print("case overlap N=%d count=%d shift=%s own=%s" % (n, count, shift, own), flush=True)
+    P = n ** 3
+    buf = torch.empty((count + 6) * P, dtype=torch.complex64, device="cuda")
+    api.fill_uniform(buf, 2 * buf.numel(), 70001 + n)
+    filt = torch.empty((count if own else 1, P), dtype=torch.complex64, device="cuda")
+    api.fill_uniform(filt, 2 * filt.numel(), 70002 + n)
+    try:
+        api.set_plan(n, api.CF_PLAN_SPLIT3_G24)
+        spec = gpu.Spectrum(n, filt, count if own else 1)
+    finally:
+        api.set_plan(n, api.CF_PLAN_AUTO)
+    at = 3 * P
+    to = at + int(shift * P)
+    sig, out = buf[at:at + count * P], buf[to:to + count * P]
+    want = torch.empty_like(sig)
+    gpu.conv3d_device(spec, sig, want, count)
+    gpu.conv3d_device(spec, sig, out, count)
+    assert _same(out, want)
+    spec.close()
