@@ -46,7 +46,7 @@ SUPPORTED_SIZES = (8, 16, 32, 64, 128, 256, 512)
 # names of every symbol include/convfpga/*.h declares
 DROPIN_SYMBOLS = ("fpga_initialize", "fpga_final", "fpgaf_complex_malloc", "fpgaf_conv3D",
                   "fpgaf_conv3D_svm", "fpgaf_conv3D_svm_batch")
-EXT_SYMBOLS = ("cf_last_error", "cf_supported_size", "cf_spectrum_create", "cf_spectrum_destroy",
+EXT_SYMBOLS = ("cf_last_error", "cf_supported_size", "cf_spectrum_create", "cf_trim", "cf_spectrum_destroy",
                "cf_spectrum_data", "cf_spectrum_edge", "cf_spectrum_count", "cf_spectrum_view", "cf_conv3d_device", "cf_conv3d_device_noalloc", "cf_conv3d_host",
                "cf_conv3d_device_timed", "cf_conv3d_share_timed", "cf_fft3d_device", "cf_rel_l2_device", "cf_profile_begin",
                "cf_profile_end", "cf_fill_uniform", "cf_fill_loguniform", "cf_plan_supported", "cf_set_plan", "cf_get_plan",
@@ -109,6 +109,7 @@ def lib():
             "cf_supported_size": (i, [u]),
             "cf_spectrum_create": (i, [u, u, vp, i, vp, ctypes.POINTER(vp)]),
             "cf_spectrum_destroy": (None, [vp]),
+            "cf_trim": (i, []),
             "cf_spectrum_data": (vp, [vp]),
             "cf_spectrum_edge": (u, [vp]),
             "cf_spectrum_count": (u, [vp]),
@@ -324,6 +325,12 @@ class Spectrum:
             self.close()
         except Exception:
             pass
+
+
+def trim():
+    """Gives back the device memory kept for later calls: destroyed spectra and the
+    transforms' workspaces (cf_trim); waits for the device."""
+    _check(lib().cf_trim(), "cf_trim")
 
 
 def conv3d_device(spec, sig, out, how_many=1, scale=CF_SCALE_INV_N3, precision=CF_PREC_FP32, stream=None):

@@ -1784,6 +1784,16 @@ extern "C" int cf_spectrum_view(cf_spectrum_t parent, unsigned index, cf_spectru
   return CF_OK;
 }
 
+extern "C" int cf_trim(void) {
+  std::lock_guard<std::recursive_mutex> lk(g.mu);
+  CFCHK(require_ready());
+  HIPCHK(hipDeviceSynchronize());
+  spec_pool_shrink(0, 0);
+  for (FftWork& w : g.fft_work) (void)hipFree(w.d);
+  g.fft_work.clear();
+  return CF_OK;
+}
+
 extern "C" const void* cf_spectrum_data(cf_spectrum_t h) {
   std::lock_guard<std::recursive_mutex> lk(g.mu);
   if (!h) return nullptr;

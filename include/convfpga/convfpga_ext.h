@@ -118,6 +118,11 @@ typedef struct cf_spectrum_s *cf_spectrum_t;
 int cf_spectrum_create(unsigned N, unsigned count, const void *filters, int on_device, void *stream,
                        cf_spectrum_t *out);
 void cf_spectrum_destroy(cf_spectrum_t h);
+/* Gives the device memory back that the library keeps for later calls: that of
+ * destroyed spectra and the workspaces of cf_fft3d_device (1 and 2 GiB at most).
+ * For programs that need it for themselves; waits for the device, so not while a
+ * stream is being recorded into a graph. */
+int cf_trim(void);
 /* device address of the spectra: count * N^3 complex floats, natural order for
  * CF_PLAN_AXIS5 / CF_PLAN_PLANE3, an internal blocked order for CF_PLAN_SPLIT3_*
  * and CF_PLAN_AXIS5Z */

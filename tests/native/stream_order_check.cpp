@@ -240,6 +240,33 @@ static void conv_overlap() {
         }
 }
 
+// What is kept for later calls can be given back, and is made again when needed.
+static void trim() {
+  CHECK(cf_set_plan(256, CF_PLAN_AXIS5) == CF_OK);
+  Bufs b(256);
+  cf_spectrum_t h = nullptr;
+  CHECK(cf_spectrum_create(256, 1, b.in, 1, nullptr, &h) == CF_OK);
+  const size_t held = rec::held - cube(256);
+  hipStream_t s = rec::new_stream();
+  for (int k = 0; k < 2; ++k) {
+    CHECK(fft(256, b, s) == CF_OK);
+    if (h) cf_spectrum_destroy(h);
+    h = nullptr;
+    CHECK(rec::held > held);
+    rec::begin_capture(s, hipStreamCaptureModeRelaxed);
+    rec::mode = hipStreamCaptureModeRelaxed;
+    CHECK(cf_trim() < 0 && rec::held > held);  // (refused, nothing freed)
+    rec::mode = hipStreamCaptureModeGlobal;
+    rec::end_capture(s);
+    rec::faults.clear();
+    rec::device_waits = 0;
+    CHECK(cf_trim() == CF_OK);
+    CHECK(rec::held == held && rec::device_waits > 0 && rec::faults.empty());
+  }
+  CHECK(cf_spectrum_create(256, 1, b.in, 1, nullptr, &h) == CF_OK);
+  CHECK(rec::races() == 0);
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
@@ -250,7 +277,8 @@ int main(int argc, char** argv) {
                 {"fft_first_call", fft_first_call},
                 {"conv_per_thread", conv_per_thread},
                 {"spectrum_reuse", spectrum_reuse},
-                {"conv_overlap", conv_overlap}};
+                {"conv_overlap", conv_overlap},
+                {"trim", trim}};
   CHECK(fpga_initialize("gfx950", "recorded", false) == 0);
   bool found = false;
   for (auto& c : checks)

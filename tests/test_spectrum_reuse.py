@@ -96,3 +96,28 @@ def test_old_spectrum_is_read_while_the_next_is_made(gpu, n, count, other_stream
     finally:
         api.set_plan(n, api.CF_PLAN_AUTO)
     assert torch.equal(_bits(out), _bits(want))
+
+
+def test_kept_memory_is_given_back(gpu):
+    """trim() leaves neither destroyed spectra nor transform workspaces; both are
+    made again."""
+    import torch
+    n = 256
+    print("case trim", flush=True)
+    x = torch.empty((2, n ** 3), dtype=torch.complex64, device="cuda")
+    gpu.api.fill_uniform(x, 2 * x.numel(), 68001)
+    want, out = torch.empty_like(x), torch.empty_like(x)
+
+    def calls(y):
+        gpu.fft3d_device(n, x[0], y[0])
+        spec = gpu.Spectrum(n, x[1])
+        gpu.conv3d_device(spec, x[0], y[1])
+        spec.close()
+    calls(want)
+    gpu.api.trim()
+    free0 = torch.cuda.mem_get_info()[0]
+    calls(out)
+    kept = torch.cuda.mem_get_info()[0]
+    gpu.api.trim()
+    assert free0 - kept >= 2 * 8 * n ** 3 and torch.cuda.mem_get_info()[0] >= free0
+    assert torch.equal(_bits(out), _bits(want))

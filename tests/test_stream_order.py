@@ -10,7 +10,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 CHECKS = ["fft_per_thread", "fft_streams", "fft_beside_capture", "fft_first_call", "conv_per_thread",
-          "spectrum_reuse", "conv_overlap"]
+          "spectrum_reuse", "conv_overlap", "trim"]
 
 needs_gxx = pytest.mark.skipif(shutil.which("g++") is None or not os.path.exists(os.path.join(ROCM, "include", "hip")),
                                reason="needs g++ and the HIP headers")
