@@ -152,12 +152,12 @@ struct SpecMem {
     stream = s;
   }
 };
-// Freed spectra kept for the next one of the same size.  hipMalloc and hipFree
+// Freed spectra kept for the next one of the same size on the stream.  hipMalloc and hipFree
 // of a 256^3 spectrum, with the device synchronisation of the latter, cost as
 // much as the transform and the convolution together: a convolution with a new
 // filter took 594 us at 256^3 (3.5 ms the first time) and 81 us at 64^3, with
 // kept memory 273 (285) and 34.  Oldest out first; given back when an
-// allocation fails and by fpga_final().
+// allocation fails, by cf_trim() and by fpga_final().
 constexpr size_t kSpecPoolBytes = size_t(1) << 30;
 constexpr size_t kSpecPoolBlocks = 4;
 
@@ -714,9 +714,8 @@ size_t work_bytes(int plan, unsigned n, unsigned nb, const void* sig, const void
 
 // Filter setup of `plan`: the forward FFT3 of `count` filters into dst, in the
 // layout the plan's product pass reads (in place when src == dst).  Natural
-// order by the axis passes (PLANE3: the plane pass and z); z-blocked for
-// AXIS5Z; for the four-step plans the
-// first pass of the convolution into the workspace, then the forward half of
+// order by the passes of the plain transform (fwd_passes); z-blocked for AXIS5Z;
+// for the four-step plans the first pass of the convolution into the workspace, then the forward half of
 // the middle pass straight into the middle pass's spectrum order (4 volume
 // transfers instead of 6 for the axis passes and 2 for a re-layout).
 void spectrum_passes(const SizeFns& f, int plan, unsigned n, unsigned count, const void* src, void* dst, void* work,
@@ -785,10 +784,11 @@ int run_passes(const PassList& v, unsigned n, unsigned nb, hipStream_t s, const 
 // How many of `count` cubes of edge n go through a schedule's passes together:
 // evenly sized groups of at most about kGroupBytes of cubes.  The next pass then
 // finds what a pass wrote in the 256 MiB memory-side cache.  Passes over the whole
-// batch against groups (us per call): 4 x 256^3 own filters 752 -> 648, split-FP16
-// 920 -> 812; 40 x 128^3 824 -> 786 in groups of 8 (854 in groups of 4, whose passes
-// no longer fill the GPU); 300 x 64^3 721 -> 637 in groups of 75 (783 of 16); 4
-// transforms of 256^3 651 -> 535.  A group may be larger by `slack` eighths, where
+// batch against groups (us per call, own filters / one filter): 4 x 256^3 797 / 798 ->
+// 630 / 631, split-FP16 888 -> 720 (own); 40 x 128^3 1027 / 887 -> 775 / 755 in groups of
+// 8 (845 / 833 of 4, whose passes no longer fill the GPU); 300 x 64^3 818 / 718 -> 710 /
+// 619 in groups of 60 / 75 (757 / 636 of 34 / 43, 855 / 715 of 18 / 22); transforms 4 x 256^3 447 -> 391,
+// 40 x 128^3 494 -> 478, 300 x 64^3 480 -> 421.  A group may be larger by `slack` eighths, where
 // two smaller ones gain less from the cache than they lose (us per cube): 64^3 own
 // filters 40: 2.42, 64: 2.36, 72: 2.38, 80: 2.52, 127: 2.68, shared 40: 2.15, 64: 2.08,
 // 88: 2.08, 96: 2.13, transforms 40: 1.44, 88: 1.42, 127: 1.57; 128^3 own 5: 20.5, 8:

@@ -13,7 +13,8 @@
 // For one cube, whose passes are three launches of a few microseconds bound by
 // one tile's chain of loads, exchanges and stores: the plane passes run 64
 // work-groups of 512 threads (a quarter of the CUs), these 128 of 256 and 256 of
-// 128, with shorter chains: 13.4 -> 12.3 us per convolution.  Batches fill the
+// 128, with shorter chains: 13.3 -> 12.4 us per convolution on one signal, 13.8 ->
+// 12.3 on 2 GiB of them in turn, 14.3 -> 13.7 with a filter each.  Batches fill the
 // GPU with planes and move whole lines in every pass: 2 cubes 15.9 us with the
 // plane passes against 16.3, 16 cubes 44.5 against 68; wider middle tiles (4, 8,
 // 16 x) come level at 4 to 8 cubes and lose above.

@@ -7,8 +7,8 @@
 // three axes are turned into each other through LDS.  As five axis passes
 // (x, y, z*H*z, y^-1, x^-1), such a cube is five launches whose kernels each
 // take 2-3 us for 64 KiB of traffic; here it is one: back-to-back calls on one
-// 16^3 cube 16.7 -> 6.0 us each.  What bounds it is the launch and the chain of
-// one work-group (load, six transforms, five exchanges, store).  The lines are
+// 16^3 cube 15.7 -> 6.0 us each.  What bounds it is the launch and the chain of
+// one work-group (load, six transforms, six exchanges, store).  The lines are
 // transformed in the order of the axis passes with the same DFT code, so the
 // results are the same bits.
 #pragma once

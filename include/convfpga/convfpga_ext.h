@@ -112,8 +112,8 @@ int cf_autotune(unsigned N, float *ms);
  * recorded call used, or whose address was taken, and then waits for the device.
  * Otherwise it does not wait for convolutions still queued with the spectrum:
  * its memory is kept for later spectra of the size made on the same stream (four
- * at most, 1 GiB in all) until an allocation of this library needs it or
- * fpga_final(). */
+ * at most, 1 GiB in all) until an allocation of this library needs it, cf_trim()
+ * or fpga_final(). */
 typedef struct cf_spectrum_s *cf_spectrum_t;
 int cf_spectrum_create(unsigned N, unsigned count, const void *filters, int on_device, void *stream,
                        cf_spectrum_t *out);
@@ -140,7 +140,12 @@ int cf_spectrum_view(cf_spectrum_t parent, unsigned index, cf_spectrum_t *out);
 
 /* ---- device-resident convolution --------------------------------------------
  * how_many cubes d_sig -> d_out (may be the same buffer).  With a spectrum of
- * count 1 every cube uses it; with count == how_many cube b uses spectrum b. */
+ * count 1 every cube uses it; with count == how_many cube b uses spectrum b.
+ * Plans with an intermediate share one workspace of the library between all
+ * streams: a call on another stream than the last one's waits for what that
+ * stream, which must still exist, holds by then.  Not for a stream that is being
+ * recorded into a graph (cf_conv3d_device_noalloc, or a batch, is), nor on
+ * another one while the last call's stream is. */
 int cf_conv3d_device(cf_spectrum_t h, const void *d_sig, void *d_out, unsigned how_many, int scale_mode,
                      int precision, void *stream);
 
@@ -263,7 +268,7 @@ int cf_batch_create_stall_test(const cf_instance_t *inst, unsigned count, int sc
 /* forward (inverse = 0) or unnormalised inverse (inverse = 1) 3D FFT.  Calls on
  * different streams are independent of each other.  N = 256 and 512 go through
  * a workspace (128 and 256 MiB) that belongs to the stream, made by its first
- * such call and kept until fpga_final(), 2 GiB in all; calls on further streams,
+ * such call and kept until cf_trim() or fpga_final(), 2 GiB in all; calls on further streams,
  * on hipStreamPerThread, or recorded into a graph run one pass per axis without
  * it (at N = 256 the two routes round differently). */
 int cf_fft3d_device(unsigned N, const void *d_in, void *d_out, unsigned how_many, int inverse, void *stream);
