@@ -143,9 +143,10 @@ int cf_spectrum_view(cf_spectrum_t parent, unsigned index, cf_spectrum_t *out);
  * count 1 every cube uses it; with count == how_many cube b uses spectrum b.
  * Plans with an intermediate share one workspace of the library between all
  * streams: a call on another stream than the last one's waits for what that
- * stream, which must still exist, holds by then.  Not for a stream that is being
- * recorded into a graph (cf_conv3d_device_noalloc, or a batch, is), nor on
- * another one while the last call's stream is. */
+ * stream, which must still exist and not be recording a graph, holds by then.  A
+ * call that is itself recorded has the workspace's address in the graph, and its
+ * replays are ordered with nothing: cf_conv3d_device_noalloc and the batches are
+ * the calls for graphs. */
 int cf_conv3d_device(cf_spectrum_t h, const void *d_sig, void *d_out, unsigned how_many, int scale_mode,
                      int precision, void *stream);
 
